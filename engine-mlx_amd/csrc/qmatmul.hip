@@ -38,62 +38,10 @@
 // past its range read zeros out of bounds instead of branching. For larger M (when the
 // dequantising GEMM does not apply) the row tiles of one weight tile are dispatched
 // together on one XCD, so its L2 serves the re-reads.
-#include "ema_common.hpp"
+#include "qmatmul_common.hpp"
 
 namespace ema {
 namespace {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-constexpr int kMaxWaves = 8;
-constexpr uint32_t kOffRow = 0xF0000000u;  // a buffer offset past every range: loads return 0
-
-struct QmmArgs {
-  const uint8_t* x;  // [M, ldx] activations
-  const uint8_t* w;  // [N, K * BITS / 8] packed fields
-  const uint8_t* s;  // [N, G] scales
-  const uint8_t* b;  // [N, G] biases
-  uint8_t* y;        // [M, ldy]
-  int64_t ldx, ldy;  // row strides in elements
-  int M, N, K, G;    // G = K / GS
-  int mtiles;        // row tiles of x (16 * MR rows each)
-  int remap;         // grid size divisible by 8: give each XCD a contiguous range of tiles
-};
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
-
-template <bool F16>
-__device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
-  if constexpr (F16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
-                                                  0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                   0, 0, 0);
-}
-
-template <bool F16>
-__device__ __forceinline__ float act_to_f32(uint32_t bits16) {
-  if constexpr (F16)
-    return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16);
-  else
-    return __uint_as_float(bits16 << 16);
-}
-template <bool F16>
-__device__ __forceinline__ uint16_t f32_to_act(float v) {
-  if constexpr (F16)
-    return __builtin_bit_cast(uint16_t, (_Float16)v);
-  else
-    return (uint16_t)f32_to_bf16_bits(v);
-}
-
-// v_perm_b32 selectors: {lo16(lo), lo16(hi)} and {hi16(lo), hi16(hi)} of two dwords.
-constexpr uint32_t kSelLo = 0x05040100u, kSelHi = 0x07060302u;
-__device__ __forceinline__ uint32_t pair(uint32_t lo, uint32_t hi, uint32_t sel) {
-  return __builtin_amdgcn_perm(hi, lo, sel);
-}
 
 // (x & m) | c in one v_and_or_b32. gfx950's VOP3 encoding takes no 32-bit literal, so with
 // literal masks the compiler splits it into v_and + v_or; the empty asm statements hand the
@@ -791,9 +739,6 @@ struct DqPlan {
   int rm, rn;  // tile rows / columns per region (regions: mtiles / rm x ntiles / rn = 8), or 0
 };
 
-// byte I of x as f32 (v_cvt_f32_ubyteI)
-template <int I>
-__device__ __forceinline__ float ubyte_f32(uint32_t x) { return (float)((x >> (8 * I)) & 0xFFu); }
 __device__ __forceinline__ uint32_t dq_unit(uint32_t row, uint32_t u) { return row * 8 + (u ^ ((row >> 1) & 7)); }
 // Buffer loads issued as asm, untracked by the compiler: the loader waits for them with
 // explicit vmcnt counts (a wait that takes the loaded registers as operands, so that no use
@@ -891,32 +836,9 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
       uint8_t* const wb = xb + kDqXBytes;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {  // unit 2 wh + u: k 8 u .. 8 u + 7 of the quarter
-        float q[8];
-        if constexpr (BITS == 4) {
-          const uint32_t wd = r.w[u], lo = wd & 0x0F0F0F0Fu, hi = (wd >> 4) & 0x0F0F0F0Fu;  // fields 2i, 2i + 1
-          q[0] = ubyte_f32<0>(lo);
-          q[1] = ubyte_f32<0>(hi);
-          q[2] = ubyte_f32<1>(lo);
-          q[3] = ubyte_f32<1>(hi);
-          q[4] = ubyte_f32<2>(lo);
-          q[5] = ubyte_f32<2>(hi);
-          q[6] = ubyte_f32<3>(lo);
-          q[7] = ubyte_f32<3>(hi);
-        } else {
-          q[0] = ubyte_f32<0>(r.w[2 * u]);
-          q[1] = ubyte_f32<1>(r.w[2 * u]);
-          q[2] = ubyte_f32<2>(r.w[2 * u]);
-          q[3] = ubyte_f32<3>(r.w[2 * u]);
-          q[4] = ubyte_f32<0>(r.w[2 * u + 1]);
-          q[5] = ubyte_f32<1>(r.w[2 * u + 1]);
-          q[6] = ubyte_f32<2>(r.w[2 * u + 1]);
-          q[7] = ubyte_f32<3>(r.w[2 * u + 1]);
-        }
         u32x4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          o[e] = (uint32_t)f32_to_act<F16>(__builtin_fmaf(sc, q[2 * e], bc)) |
-                 ((uint32_t)f32_to_act<F16>(__builtin_fmaf(sc, q[2 * e + 1], bc)) << 16);
+        if constexpr (BITS == 4) o = dequant8<BITS, F16>(r.w[u], 0u, sc, bc);
+        else o = dequant8<BITS, F16>(r.w[2 * u], r.w[2 * u + 1], sc, bc);
         *reinterpret_cast<u32x4*>(wb + 16 * dq_unit(wr_row, 2 * wh + u)) = o;
       }
     };
@@ -1190,6 +1112,8 @@ int32_t launch_t(hipStream_t st, QmmArgs a) {
     }
     if (p.NC > 0) return launch_qmv_rows<BITS, GS, F16>(st, a, mx, p);
   } else {
+    const KsPlan kp = plan_ks(a, GS, BITS, cus);
+    if (kp.mt > 0) return launch_qgemm_ks(st, a, kp, GS, BITS, F16);
     DqPlan dp;
     if (plan_dq(a.M, a.N, a.K, GS, BITS, a.ldx, &dp)) return launch_dq<BITS, GS, F16>(st, a, dp);
   }

@@ -160,6 +160,39 @@ def test_qmatmul_prefill_rows(ema, ora, M, N, K, gs, bits, dtype):
     check(ora, y, h, gs, bits, f"M={M}", dtype)
 
 
+@pytest.mark.parametrize("M,N,K,gs,bits,dtype", [
+    # the K-split GEMM: each of its tiles (row x column tiles of 16, chosen by the number of
+    # tiles on 256 CUs), ragged last rows and columns, fewer units of 128 k than waves
+    (33, 100, 128, 32, 4, "bf16"),      # 3 x 2, one unit
+    (48, 30, 384, 32, 8, "f16"),        # 3 x 2, three units
+    (64, 5100, 256, 64, 4, "f16"),      # 4 x 2
+    (157, 4093, 256, 64, 4, "bf16"),    # 5 x 2
+    (157, 4090, 512, 128, 8, "bf16"),   # 5 x 2
+    (96, 6140, 256, 64, 8, "bf16"),     # 3 x 3
+    (101, 6144, 256, 32, 4, "bf16"),    # 4 x 3
+    (127, 6143, 256, 32, 8, "f16"),     # 4 x 3
+    (159, 6142, 512, 128, 4, "f16"),    # 5 x 3
+    (140, 5437, 256, 64, 4, "bf16"),    # 3 x 4
+    (140, 5440, 256, 64, 8, "f16"),     # 3 x 4
+    (190, 5439, 256, 32, 4, "bf16"),    # 4 x 4
+    (80, 64, 1152, 64, 4, "bf16"),      # nine units: one wave takes two
+    (50, 70, 2560, 64, 8, "bf16"),      # twenty units
+])
+def test_qmatmul_ksplit_tiles(ema, ora, M, N, K, gs, bits, dtype):
+    import torch
+
+    say(f"qmatmul K-split M={M} N={N} K={K} gs={gs} bits={bits} {dtype}")
+    d, h = make(ora, M + N + K, M, N, K, gs, bits, dtype)
+    y = ema.quantized_matmul(*d, group_size=gs, bits=bits)
+    check(ora, y, h, gs, bits, f"M={M}", dtype)
+    # into a view with an odd row stride (2-byte stores): the same bits, nothing beside them
+    wide = torch.full((M, N + 3), 7.0, dtype=y.dtype, device="cuda")
+    ema.quantized_matmul(*d, group_size=gs, bits=bits, out=wide[:, 1:N + 1])
+    torch.cuda.synchronize()
+    assert torch.equal(wide[:, 1:N + 1].contiguous().view(torch.int16), y.view(torch.int16))
+    assert torch.all(wide[:, :1] == 7.0) and torch.all(wide[:, N + 1:] == 7.0)
+
+
 @pytest.mark.parametrize("M", [1, 32, 256])
 def test_qmatmul_graph_replay(ema, ora, M):
     # captured in a HIP graph and replayed several times with eager work between the

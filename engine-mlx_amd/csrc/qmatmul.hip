@@ -13,9 +13,11 @@
 //
 // Two regimes, as in MLX, whose quantized matmul takes vector kernels for a few rows of x
 // and, for many, kernels that dequantise weight tiles into the activation type first:
-// - up to 32 rows (and the streaming fallback): exact products, below;
-// - more than 32 rows with K a multiple of 64: qgemm_dq_kernel, on weights dequantised
-//   into bf16 / f16 (one rounding each) in LDS.
+// - up to 32 rows (and the streaming fallback): exact products, below, and qgemm_ks.hip from
+//   K = 2048 on;
+// - more than 32 rows with K a multiple of 64: qgemm_dq_kernel, and the K-split kernel of
+//   qgemm_ks.hip where small tiles fill the chip better, on weights dequantised into bf16 /
+//   f16 (one rounding each).
 //
 // Exact products. The MFMA's B operand is not the dequantised weight (which would have to
 // be rounded to bf16) but C + q, with the field's bits dropped into the mantissa of the
@@ -42,77 +44,6 @@
 
 namespace ema {
 namespace {
-
-// (x & m) | c in one v_and_or_b32. gfx950's VOP3 encoding takes no 32-bit literal, so with
-// literal masks the compiler splits it into v_and + v_or; the empty asm statements hand the
-// constants over as VGPR values (set once per kernel) and the compiler selects the fused
-// instruction. The instruction itself is left to the compiler: its result feeds MFMA
-// operands, and the hazard recognizer inserts the wait states a VALU write needs before an
-// MFMA reads it only for instructions it emits itself, not for an inline-asm VALU
-// instruction.
-__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t m, uint32_t c) {
-  asm("" : "+v"(m));
-  asm("" : "+v"(c));
-  return (x & m) | c;
-}
-
-template <int BITS, bool F16>
-struct Fields {
-  // the weight bits take the mantissa of this constant: value kOff + q, exact
-  static constexpr bool kMagic = F16 || BITS == 4;
-  static constexpr uint32_t kMagicBits = F16 ? 0x64006400u : 0x43004300u;  // 1024 (f16), 128 (bf16)
-  static constexpr float kOff = !kMagic ? 0.0f : (F16 ? 1024.0f : 128.0f);
-  static constexpr uint32_t kOnes = F16 ? 0x3C003C00u : 0x3F803F80u;
-
-  // B operand of MFMA step `st`: 8 fields of this lane's weight dwords.
-  static __device__ __forceinline__ u32x4 weights(const uint32_t* wd, int st) {
-    u32x4 r;
-    if constexpr (BITS == 4) {
-      const uint32_t w = wd[st];  // fields 0..7; register i holds fields i and i + 4
-      r[0] = and_or(w, 0x000F000Fu, kMagicBits);
-      r[1] = and_or(w >> 4, 0x000F000Fu, kMagicBits);
-      r[2] = and_or(w >> 8, 0x000F000Fu, kMagicBits);
-      r[3] = and_or(w >> 12, 0x000F000Fu, kMagicBits);
-    } else if constexpr (F16) {
-      const uint32_t w0 = wd[2 * st], w1 = wd[2 * st + 1];  // bytes 0..3, 4..7
-      r[0] = and_or(w0, 0x00FF00FFu, kMagicBits);           // bytes 0, 2
-      r[1] = and_or(w0 >> 8, 0x00FF00FFu, kMagicBits);      // bytes 1, 3
-      r[2] = and_or(w1, 0x00FF00FFu, kMagicBits);
-      r[3] = and_or(w1 >> 8, 0x00FF00FFu, kMagicBits);
-    } else {
-      const uint32_t w0 = wd[2 * st], w1 = wd[2 * st + 1];
-      // an integer below 256 is exact in the top half of its f32
-      const uint32_t f0 = __float_as_uint((float)(w0 & 0xFFu)), f1 = __float_as_uint((float)((w0 >> 8) & 0xFFu));
-      const uint32_t f2 = __float_as_uint((float)((w0 >> 16) & 0xFFu)), f3 = __float_as_uint((float)(w0 >> 24));
-      const uint32_t f4 = __float_as_uint((float)(w1 & 0xFFu)), f5 = __float_as_uint((float)((w1 >> 8) & 0xFFu));
-      const uint32_t f6 = __float_as_uint((float)((w1 >> 16) & 0xFFu)), f7 = __float_as_uint((float)(w1 >> 24));
-      r[0] = pair(f0, f1, kSelHi);
-      r[1] = pair(f2, f3, kSelHi);
-      r[2] = pair(f4, f5, kSelHi);
-      r[3] = pair(f6, f7, kSelHi);
-    }
-    return r;
-  }
-  // A operand of the same step: 8 consecutive activations (4 dwords) paired as the
-  // fields above are.
-  static __device__ __forceinline__ u32x4 acts(const uint32_t* d) {
-    u32x4 r;
-    if constexpr (BITS == 4) {  // {x_i, x_i+4}
-      r[0] = pair(d[0], d[2], kSelLo);
-      r[1] = pair(d[0], d[2], kSelHi);
-      r[2] = pair(d[1], d[3], kSelLo);
-      r[3] = pair(d[1], d[3], kSelHi);
-    } else if constexpr (F16) {  // {x_0, x_2}, {x_1, x_3}, {x_4, x_6}, {x_5, x_7}
-      r[0] = pair(d[0], d[1], kSelLo);
-      r[1] = pair(d[0], d[1], kSelHi);
-      r[2] = pair(d[2], d[3], kSelLo);
-      r[3] = pair(d[2], d[3], kSelHi);
-    } else {
-      r = u32x4{d[0], d[1], d[2], d[3]};
-    }
-    return r;
-  }
-};
 
 // Loads N dwords (1, 2 or a multiple of 4) at byte offset `off` of buffer `r`.
 template <int N>
@@ -1095,6 +1026,8 @@ int32_t launch_t(hipStream_t st, QmmArgs a) {
   const int cus = device_cus();
   if (a.M == 1 && gemv1_fits(a.G, a.K)) return launch_gemv1<BITS, GS, F16>(st, a, cus);
   if (a.M <= 32) {
+    const KsPlan kp = plan_qmv_ks(a, cus);
+    if (kp.mt > 0) return launch_qmv_ks(st, a, kp, GS, BITS, F16);
     const int mx = qmv_rows(a.M);
     const QmvPlan p = plan_qmv(a.N, a.K, GS, BITS, mx, cus);
     if (mx >= 16) {
@@ -1112,7 +1045,7 @@ int32_t launch_t(hipStream_t st, QmmArgs a) {
     }
     if (p.NC > 0) return launch_qmv_rows<BITS, GS, F16>(st, a, mx, p);
   } else {
-    const KsPlan kp = plan_ks(a, GS, BITS, cus);
+    const KsPlan kp = plan_ks(a, BITS, cus);
     if (kp.mt > 0) return launch_qgemm_ks(st, a, kp, GS, BITS, F16);
     DqPlan dp;
     if (plan_dq(a.M, a.N, a.K, GS, BITS, a.ldx, &dp)) return launch_dq<BITS, GS, F16>(st, a, dp);

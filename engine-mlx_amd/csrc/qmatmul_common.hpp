@@ -21,8 +21,11 @@ struct QmmArgs {
 struct KsPlan {
   int mt, nt;
 };
-KsPlan plan_ks(const QmmArgs& a, int gs, int bits, int cus);
+KsPlan plan_ks(const QmmArgs& a, int bits, int cus);
 int32_t launch_qgemm_ks(hipStream_t st, const QmmArgs& a, const KsPlan& p, int gs, int bits, bool f16);
+// The same for the exact products of up to 32 rows.
+KsPlan plan_qmv_ks(const QmmArgs& a, int cus);
+int32_t launch_qmv_ks(hipStream_t st, const QmmArgs& a, const KsPlan& p, int gs, int bits, bool f16);
 
 namespace {
 
@@ -117,6 +120,77 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t w0, uint32_t w1, float sc, fl
     o[e] = pack_act2<F16>(__builtin_fmaf(sc, q[2 * e], bc), __builtin_fmaf(sc, q[2 * e + 1], bc));
   return o;
 }
+
+// (x & m) | c in one v_and_or_b32. gfx950's VOP3 encoding takes no 32-bit literal, so with
+// literal masks the compiler splits it into v_and + v_or; the empty asm statements hand the
+// constants over as VGPR values (set once per kernel) and the compiler selects the fused
+// instruction. The instruction itself is left to the compiler: its result feeds MFMA
+// operands, and the hazard recognizer inserts the wait states a VALU write needs before an
+// MFMA reads it only for instructions it emits itself, not for an inline-asm VALU
+// instruction.
+__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t m, uint32_t c) {
+  asm("" : "+v"(m));
+  asm("" : "+v"(c));
+  return (x & m) | c;
+}
+
+template <int BITS, bool F16>
+struct Fields {
+  // the weight bits take the mantissa of this constant: value kOff + q, exact
+  static constexpr bool kMagic = F16 || BITS == 4;
+  static constexpr uint32_t kMagicBits = F16 ? 0x64006400u : 0x43004300u;  // 1024 (f16), 128 (bf16)
+  static constexpr float kOff = !kMagic ? 0.0f : (F16 ? 1024.0f : 128.0f);
+  static constexpr uint32_t kOnes = F16 ? 0x3C003C00u : 0x3F803F80u;
+
+  // B operand of MFMA step `st`: 8 fields of this lane's weight dwords.
+  static __device__ __forceinline__ u32x4 weights(const uint32_t* wd, int st) {
+    u32x4 r;
+    if constexpr (BITS == 4) {
+      const uint32_t w = wd[st];  // fields 0..7; register i holds fields i and i + 4
+      r[0] = and_or(w, 0x000F000Fu, kMagicBits);
+      r[1] = and_or(w >> 4, 0x000F000Fu, kMagicBits);
+      r[2] = and_or(w >> 8, 0x000F000Fu, kMagicBits);
+      r[3] = and_or(w >> 12, 0x000F000Fu, kMagicBits);
+    } else if constexpr (F16) {
+      const uint32_t w0 = wd[2 * st], w1 = wd[2 * st + 1];  // bytes 0..3, 4..7
+      r[0] = and_or(w0, 0x00FF00FFu, kMagicBits);           // bytes 0, 2
+      r[1] = and_or(w0 >> 8, 0x00FF00FFu, kMagicBits);      // bytes 1, 3
+      r[2] = and_or(w1, 0x00FF00FFu, kMagicBits);
+      r[3] = and_or(w1 >> 8, 0x00FF00FFu, kMagicBits);
+    } else {
+      const uint32_t w0 = wd[2 * st], w1 = wd[2 * st + 1];
+      // an integer below 256 is exact in the top half of its f32
+      const uint32_t f0 = __float_as_uint((float)(w0 & 0xFFu)), f1 = __float_as_uint((float)((w0 >> 8) & 0xFFu));
+      const uint32_t f2 = __float_as_uint((float)((w0 >> 16) & 0xFFu)), f3 = __float_as_uint((float)(w0 >> 24));
+      const uint32_t f4 = __float_as_uint((float)(w1 & 0xFFu)), f5 = __float_as_uint((float)((w1 >> 8) & 0xFFu));
+      const uint32_t f6 = __float_as_uint((float)((w1 >> 16) & 0xFFu)), f7 = __float_as_uint((float)(w1 >> 24));
+      r[0] = pair(f0, f1, kSelHi);
+      r[1] = pair(f2, f3, kSelHi);
+      r[2] = pair(f4, f5, kSelHi);
+      r[3] = pair(f6, f7, kSelHi);
+    }
+    return r;
+  }
+  // A operand of the same step: 8 consecutive activations (4 dwords) paired as the
+  // fields above are.
+  static __device__ __forceinline__ u32x4 acts(const uint32_t* d) {
+    u32x4 r;
+    if constexpr (BITS == 4) {  // {x_i, x_i+4}
+      r[0] = pair(d[0], d[2], kSelLo);
+      r[1] = pair(d[0], d[2], kSelHi);
+      r[2] = pair(d[1], d[3], kSelLo);
+      r[3] = pair(d[1], d[3], kSelHi);
+    } else if constexpr (F16) {  // {x_0, x_2}, {x_1, x_3}, {x_4, x_6}, {x_5, x_7}
+      r[0] = pair(d[0], d[1], kSelLo);
+      r[1] = pair(d[0], d[1], kSelHi);
+      r[2] = pair(d[2], d[3], kSelLo);
+      r[3] = pair(d[2], d[3], kSelHi);
+    } else {
+      r = u32x4{d[0], d[1], d[2], d[3]};
+    }
+    return r;
+  }
+};
 
 }  // namespace
 }  // namespace ema

@@ -193,6 +193,34 @@ def test_qmatmul_ksplit_tiles(ema, ora, M, N, K, gs, bits, dtype):
     assert torch.all(wide[:, :1] == 7.0) and torch.all(wide[:, N + 1:] == 7.0)
 
 
+@pytest.mark.parametrize("M,N,K,gs,bits,dtype", [
+    # exact products split over K (K >= 2048): 8, 16 and 32 rows, one and two column tiles,
+    # ragged columns, units that do not divide among the eight waves
+    (2, 70, 2048, 64, 4, "bf16"),
+    (8, 33, 2176, 32, 4, "f16"),        # 17 units
+    (9, 100, 2048, 128, 8, "bf16"),
+    (16, 4099, 2048, 64, 4, "bf16"),    # two column tiles, ragged
+    (17, 48, 2560, 64, 8, "f16"),       # 20 units
+    (31, 4110, 2304, 32, 4, "bf16"),    # two column tiles, 18 units
+    (32, 8200, 2048, 64, 4, "bf16"),    # more than two rounds: one column tile
+    (5, 4097, 4608, 64, 8, "bf16"),     # 36 units: a fifth turn for four waves
+    (3, 40, 12288, 32, 4, "bf16"),      # 384 groups: past the LDS bound, the staged kernels
+    (4, 40, 9728, 32, 4, "f16"),        # 304 groups: scales staged in two passes
+])
+def test_qmatmul_ksplit_decode_rows(ema, ora, M, N, K, gs, bits, dtype):
+    import torch
+
+    say(f"qmatmul K-split decode M={M} N={N} K={K} gs={gs} bits={bits} {dtype}")
+    d, h = make(ora, M + N + K, M, N, K, gs, bits, dtype)
+    y = ema.quantized_matmul(*d, group_size=gs, bits=bits)
+    check(ora, y, h, gs, bits, f"M={M}", dtype)
+    wide = torch.full((M, N + 3), 7.0, dtype=y.dtype, device="cuda")
+    ema.quantized_matmul(*d, group_size=gs, bits=bits, out=wide[:, 1:N + 1])
+    torch.cuda.synchronize()
+    assert torch.equal(wide[:, 1:N + 1].contiguous().view(torch.int16), y.view(torch.int16))
+    assert torch.all(wide[:, :1] == 7.0) and torch.all(wide[:, N + 1:] == 7.0)
+
+
 @pytest.mark.parametrize("M", [1, 32, 256])
 def test_qmatmul_graph_replay(ema, ora, M):
     # captured in a HIP graph and replayed several times with eager work between the

@@ -18,9 +18,13 @@
 //     ([row block][mt][lane] f32x4);
 //   key-head record (written by the first value head of each group): the Q and K^T
 //     operand tiles.
-// gdn_wy_scan_kernel: one workgroup per (batch, value head, 64 state rows): four waves own
-// 16 state rows each, a fifth copies each chunk's records HBM -> LDS by LDS-DMA two chunks
-// ahead (three buffers). The state stays f32 in registers across the scan.
+// gdn_wy_scan_kernel: one workgroup per (batch, value head, 16, 32 or 64 state rows): its
+// waves own 16 state rows each, one more copies each chunk's records HBM -> LDS by LDS-DMA two
+// chunks ahead (three buffers). The state stays f32 in registers across the scan. Bound by
+// the chunk's chain on one wave: 62 MFMA, 229 VALU and 42 KB of operand reads. Reading every
+// operand up front took 32 heads x 2048 tokens from 121.5 to 107 us (both passes), two waves
+// per workgroup to 97, VALU issued under the MFMAs to 96; a second loader wave changed
+// nothing.
 //
 // A workspace smaller than the whole sequence is used in segments of as many chunks as
 // fit: one prep and one state pass per segment, the state passing through HBM between.
@@ -56,7 +60,8 @@ struct WyArgs {
   uint64_t v_rec;     // bytes of a value-head record
   uint64_t k_base;    // byte offset of the key-head records
   int T, hk, hv, dv;
-  int groups;         // state-pass workgroups per (batch, value head): ceil(Dv / 64)
+  int groups;         // state-pass workgroups per (batch, value head)
+  int64_t heads;      // B * Hv
   int c0, nc;         // first chunk of the segment, chunks in it
 };
 
@@ -264,8 +269,7 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0xF70);
 }
 
-constexpr int kScanWaves = 4;  // 16 state rows each, plus one loader wave
-template <int DK>
+template <int DK, int kScanWaves>
 struct ScanLds {
   static constexpr int kV = Rec<DK>::kU;        // the value-head record up to u
   static constexpr int kK = kV;                 // then the key-head record
@@ -275,18 +279,25 @@ struct ScanLds {
   static constexpr int kDma = (kBuf) / 1024;    // 1 KB steps per chunk
 };
 
-template <int DK>
-__global__ __launch_bounds__(64 * (kScanWaves + 1)) void gdn_wy_scan_kernel(WyArgs a) {
-  typedef ScanLds<DK> L;
+constexpr int kValu = 0x2, kMfma = 0x8;  // sched_group_barrier classes
+
+// kScanWaves waves of 16 state rows each, plus one loader wave
+template <int DK, int kScanWaves>
+__global__ __launch_bounds__(64 * (kScanWaves + 1)) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_wy_scan_kernel(
+    WyArgs a) {
+  typedef ScanLds<DK, kScanWaves> L;
   constexpr int S = DK / 32, NT = DK / 16;
   static_assert(L::kV % 1024 == 0 && Rec<DK>::kKey % 1024 == 0, "records move in 1 KB DMA steps");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g16 = lane & 15, c4 = lane >> 4;
-  int64_t id = blockIdx.x;
+  // the row groups of one value head on one XCD (workgroups go round the eight XCDs), so its
+  // L2 serves their shared records; the grid is rounded up to whole rounds
+  int64_t id = (int64_t)(blockIdx.x >> 3);
   const int rg = (int)(id % a.groups);
-  id /= a.groups;
+  id = id / a.groups * 8 + (blockIdx.x & 7);
+  if (id >= a.heads) return;
   const int h = (int)(id % a.hv);
   const int64_t b = id / a.hv;
   const int kh = h / (a.hv / a.hk);
@@ -359,16 +370,30 @@ __global__ __launch_bounds__(64 * (kScanWaves + 1)) void gdn_wy_scan_kernel(WyAr
       const u32x4* const KT = QA + gdnc::In<DK>::kKa;
       const f32x4* const U = (const f32x4*)(buf + L::kU) + wave * 128;
       // v = u - w S^T and Q S^T; A = -w / Q tiles, B = the state (hi + lo)
-      u32x4 w4[2][S][2], qa4[2][S];
+      // Every operand of the chunk is requested up front, in the order of use: with one wave
+      // per SIMD nothing hides an LDS round trip, and left to itself the compiler reads each
+      // operand just before its product (108 VGPRs, 28 exposed waits per chunk).
+      u32x4 w4[2][S][2], qa4[2][S], kt4[NT], qm4[4];
+      f32x4 v[2] = {U[lane], U[64 + lane]}, qs[2], gam[2], rho[2];
       #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
+      for (int s = 0; s < S; ++s)
         #pragma unroll
-        for (int s = 0; s < S; ++s) {
+        for (int mt = 0; mt < 2; ++mt) {
           w4[mt][s][0] = W[((mt * S + s) * 2 + 0) * 64 + lane];
           w4[mt][s][1] = W[((mt * S + s) * 2 + 1) * 64 + lane];
           qa4[mt][s] = QA[(mt * S + s) * 64 + lane];
         }
-      f32x4 v[2] = {U[lane], U[64 + lane]}, qs[2];
+      #pragma unroll
+      for (int mt = 0; mt < 2; ++mt) {
+        gam[mt] = *(const f32x4*)&vec[16 * mt + 4 * c4];
+        rho[mt] = *(const f32x4*)&vec[64 + 16 * mt + 4 * c4];
+      }
+      const float gc = vec[96];
+      #pragma unroll
+      for (int t = 0; t < NT; ++t) kt4[t] = KT[t * 64 + lane];
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) qm4[e] = QM[e * 64 + lane];
+      __builtin_amdgcn_sched_barrier(0);
       #pragma unroll
       for (int mt = 0; mt < 2; ++mt) qs[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
       #pragma unroll
@@ -386,20 +411,23 @@ __global__ __launch_bounds__(64 * (kScanWaves + 1)) void gdn_wy_scan_kernel(WyAr
           qs[mt] = mfma16(qa, sh, qs[mt]);
         }
       }
-      f32x4 gam[2], rho[2];
+      // the state's decay rides under the products above
       #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        gam[mt] = *(const f32x4*)&vec[16 * mt + 4 * c4];
-        rho[mt] = *(const f32x4*)&vec[64 + 16 * mt + 4 * c4];
+      for (int t = 0; t < NT; ++t) st[t] = st[t] * gc;
+      // issue order: the first split, then up to three VALU in the shadow of each MFMA
+      __builtin_amdgcn_sched_group_barrier(kValu, 24, 0);
+      #pragma unroll
+      for (int i = 0; i < 10 * S; ++i) {
+        __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kValu, 3, 0);
       }
-      const float gc = vec[96];
+      __builtin_amdgcn_sched_barrier(0);
       // S = gamma_31 S + (rho v)^T K: A = K^T tiles, B = rho v (hi + lo)
       bf16x8 th, tl;
       gdnc::split8(rho[0] * v[0], rho[1] * v[1], th, tl);
       #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const bf16x8 kt = as_bf16x8(KT[t * 64 + lane]);
-        st[t] = st[t] * gc;
+        const bf16x8 kt = as_bf16x8(kt4[t]);
         st[t] = mfma16(kt, tl, st[t]);
         st[t] = mfma16(kt, th, st[t]);
       }
@@ -413,7 +441,7 @@ __global__ __launch_bounds__(64 * (kScanWaves + 1)) void gdn_wy_scan_kernel(WyAr
           y_wave + (int64_t)t0 * y_tok, (short)0, n_tok * y_tok * 2, 0x00020000);
       #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
-        const bf16x8 qh = as_bf16x8(QM[(2 * mt) * 64 + lane]), ql = as_bf16x8(QM[(2 * mt + 1) * 64 + lane]);
+        const bf16x8 qh = as_bf16x8(qm4[2 * mt]), ql = as_bf16x8(qm4[2 * mt + 1]);
         f32x4 yv = gam[mt] * qs[mt];
         yv = mfma16(ql, vh, yv);
         yv = mfma16(qh, vl, yv);
@@ -432,16 +460,35 @@ __global__ __launch_bounds__(64 * (kScanWaves + 1)) void gdn_wy_scan_kernel(WyAr
     for (int t = 0; t < NT; ++t) *(f32x4*)(st_ptr + 16 * t) = st[t];
 }
 
+template <int DK, int kScanWaves>
+int32_t launch_scan(hipStream_t s, WyArgs a) {
+  static std::atomic<uint64_t> lds_set;
+  constexpr int kLds = ScanLds<DK, kScanWaves>::kBytes;
+  const int32_t rc = allow_lds_once((const void*)gdn_wy_scan_kernel<DK, kScanWaves>, kLds, &lds_set,
+                                    "ema_gdn_scan_ws: LDS attribute");
+  if (rc) return rc;
+  a.groups = (a.dv + 16 * kScanWaves - 1) / (16 * kScanWaves);
+  hipLaunchKernelGGL((gdn_wy_scan_kernel<DK, kScanWaves>), dim3((unsigned)((a.heads + 7) / 8 * 8 * a.groups)),
+                     dim3(64 * (kScanWaves + 1)), kLds, s, a);
+  return check_hip(hipGetLastError(), "ema_gdn_scan_ws state launch");
+}
+
 template <int DK>
 int32_t launch_wy_dk(hipStream_t s, WyArgs a, int nch, int nc_max, int B) {
-  static std::atomic<uint64_t> lds_set[2];
+  static std::atomic<uint64_t> lds_set;
   const int prep_lds = PrepLds<DK>::bytes(a.dv);
-  int32_t rc = allow_lds_once((const void*)gdn_wy_prep_kernel<DK>, PrepLds<DK>::bytes(512), &lds_set[0],
+  int32_t rc = allow_lds_once((const void*)gdn_wy_prep_kernel<DK>, PrepLds<DK>::bytes(512), &lds_set,
                               "ema_gdn_scan_ws: LDS attribute");
   if (rc) return rc;
-  rc = allow_lds_once((const void*)gdn_wy_scan_kernel<DK>, ScanLds<DK>::kBytes, &lds_set[1],
-                      "ema_gdn_scan_ws: LDS attribute");
-  if (rc) return rc;
+  // Waves (16 state rows each) per workgroup: the fewest with which the grid stays at half the
+  // CUs, else two while it stays at one workgroup per CU, else four. A workgroup of fewer waves
+  // waits less on the CU's LDS (every wave reads all of the chunk's operands), but each loads
+  // the records again. Measured, state and parallel pass, us with 1 / 2 / 4 waves: 16 heads x
+  // 3000 tokens 114 / 117 / 131; 32 x 2048 100 / 96 / 106; 64 x 1000 96 / 70 / 74; 128 x 1000
+  // 187 / 133 / 119.
+  const int cus = device_cus();
+  const int64_t g1 = a.heads * ((a.dv + 15) / 16), g2 = a.heads * ((a.dv + 31) / 32);
+  const int w = 2 * g1 <= cus ? 1 : g2 <= cus ? 2 : 4;
   for (int c0 = 0; c0 < nch; c0 += nc_max) {
     a.c0 = c0;
     a.nc = nch - c0 < nc_max ? nch - c0 : nc_max;
@@ -449,9 +496,7 @@ int32_t launch_wy_dk(hipStream_t s, WyArgs a, int nch, int nc_max, int B) {
     hipLaunchKernelGGL(gdn_wy_prep_kernel<DK>, dim3((unsigned)((int64_t)B * a.hv * a.nc)), dim3(256), prep_lds, s, a);
     rc = check_hip(hipGetLastError(), "ema_gdn_scan_ws prep launch");
     if (rc) return rc;
-    hipLaunchKernelGGL(gdn_wy_scan_kernel<DK>, dim3((unsigned)((int64_t)B * a.hv * a.groups)),
-                       dim3(64 * (kScanWaves + 1)), ScanLds<DK>::kBytes, s, a);
-    rc = check_hip(hipGetLastError(), "ema_gdn_scan_ws state launch");
+    rc = w == 1 ? launch_scan<DK, 1>(s, a) : w == 2 ? launch_scan<DK, 2>(s, a) : launch_scan<DK, 4>(s, a);
     if (rc) return rc;
   }
   return EMA_OK;
@@ -491,7 +536,8 @@ int32_t launch_gdn_wy(hipStream_t s, const void* q, const void* k, const void* v
   a.hk = hk;
   a.hv = hv;
   a.dv = dv;
-  a.groups = (dv + 63) / 64;
+  a.groups = 0;
+  a.heads = (int64_t)B * hv;
   a.c0 = 0;
   a.nc = 0;
   const int nc_max = fit < (uint64_t)nch ? (int)fit : nch;

@@ -231,6 +231,21 @@ def test_gdn_wy_scan_matches_oracle(ema, ora, T, Dk, Dv):
     check_against_oracle(ora, y, dS, host_in, "bf16", f"WY T={T} Dk={Dk} Dv={Dv}")
 
 
+@pytest.mark.parametrize("B,T,Hk,Hv,Dk,Dv", [
+    (1, 40, 1, 3, 128, 48),     # one wave per workgroup, heads not a multiple of the XCDs
+    (3, 70, 2, 10, 128, 128),   # two: 30 heads x 4 row groups
+    (7, 33, 3, 9, 64, 80),      # two: 63 heads x 3, the last row group half empty
+    (5, 65, 5, 15, 128, 112),   # four: 75 heads x 2, ragged rows
+])
+def test_gdn_wy_row_splits(ema, ora, B, T, Hk, Hv, Dk, Dv):
+    # the state pass with one, two and four waves per workgroup (chosen by the grid on 256 CUs)
+    say(f"gdn WY row split B={B} T={T} Hk={Hk} Hv={Hv} Dk={Dk} Dv={Dv}")
+    dev_in, host_in = make_inputs(700 + T, B, T, Hk, Hv, Dk, Dv, "bf16")
+    dq, dk_, dv_, dg, db, dS = dev_in
+    y = ema.gdn_scan(dq, dk_, dv_, dg, db, dS, workspace=ema.gdn_workspace(B, T, Hk, Hv, Dk, Dv))
+    check_against_oracle(ora, y, dS, host_in, "bf16", f"row split B={B} Hv={Hv} Dv={Dv}")
+
+
 def test_gdn_wy_segments_are_bit_identical(ema):
     # a workspace of 1 or 3 chunks runs the sequence in segments, the state passing through
     # HBM between them: the same arithmetic as one segment, so the same bits

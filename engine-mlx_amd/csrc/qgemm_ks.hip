@@ -60,8 +60,6 @@ __device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {
 // wave as many rows as its lanes cover; groups past 256 (long K) follow in a loop. Staged
 // before the first weights and x are requested: requesting those in between, ahead of the LDS
 // writes, took 0.2 to 0.3 us more at up to 16 rows.
-__device__ __host__ __forceinline__ uint32_t group_stride(uint32_t G) { return ((G >> 2) | 1) << 2; }
-
 template <int NT>
 struct GroupStage {
   static constexpr int kRows = 16 * NT, kPer = kRows / kKsWaves;
@@ -599,22 +597,22 @@ bool ks_fits(const QmmArgs& a) {
 
 // The tile, or mt = 0 when qgemm_dq_kernel is the better kernel or this one does not apply.
 // One workgroup per CU at a time, so a call takes rounds * time of a workgroup; measured at K
-// = 2048 and 4096, in units of 50 ns: a workgroup takes 70 and, per turn of its eight waves
-// over a unit each, 2 + 8 per row tile + 9 per column tile; one of qgemm_dq_kernel 80 + 16
-// per 64 k. (N = 4096, K = 4096: this kernel 47 us against 57 at 520 rows; N = 6144: 63
-// against 57.)
+// = 2048 and 4096, in units of 25 ns: a workgroup takes 140 and, per turn of its eight waves
+// over a unit each, 4 + 16 per row tile + 18 per column tile (qgemm_dq_kernel: dq_cost; K =
+// 4096, N = 4096: 33 us here against 45 at 300 rows, 45 against 45 at 520, 58 against 46 at
+// 700).
 KsPlan plan_ks(const QmmArgs& a, int bits, int cus) {
   KsPlan best{0, 0};
   if (!ks_fits(a)) return best;
   auto rounds = [&](int rows, int cols) {
     return (((int64_t)a.M + rows - 1) / rows * (((int64_t)a.N + cols - 1) / cols) + cus - 1) / cus;
   };
-  int64_t cost = rounds(256, 128) * (80 + 16 * (int64_t)(a.K / 64));
+  int64_t cost = dq_cost(a.M, a.N, a.K, dq_row_tiles(a.M, a.N, a.K, cus), cus);
   const int64_t turns = (a.K / kUnit + kKsWaves - 1) / kKsWaves;
   for (int mt = 3; mt <= 5; ++mt)
     for (int nt = 2; nt <= 4; ++nt) {
       if (!ks_tile(bits, mt, nt)) continue;
-      const int64_t c = rounds(16 * mt, 16 * nt) * (70 + turns * (2 + 8 * mt + 9 * nt));
+      const int64_t c = rounds(16 * mt, 16 * nt) * (140 + turns * (4 + 16 * mt + 18 * nt));
       if (c < cost) {
         cost = c;
         best = KsPlan{mt, nt};

@@ -641,18 +641,22 @@ int32_t launch_qmv_rows(hipStream_t st, const QmmArgs& a, int mx, const QmvPlan&
 // ---------------------------------------------------------------- dequantising GEMM (M > 32)
 // MLX's quantized matmul for many rows (its qmm kernels) dequantises each weight tile into
 // the activation type in threadgroup memory and multiplies that. Here likewise: a workgroup
-// owns a 256 x 128 tile of y (256 rows of x, 128 weight rows) and walks K in chunks of 64,
-// with two roles:
-// - eight compute waves, wave (wm, wn) = (wave % 4, wave / 4) multiplying its 64 x 64 block
-//   as 4 x 4 16x16x32 MFMA tiles, two k-steps per chunk, from LDS only;
-// - eight loader waves, which load each chunk's x, packed weights, scales and biases three
-//   chunks ahead into registers (three sets in turn), then write x into LDS and dequantise
-//   the weights into it, w = round(fma(s, q, b)) in f32 then to bf16 / f16 (the rounding
-//   of MLX's dequantise, parity unpinned as to one rounding or two).
+// owns a 64 MT x 128 tile of y (MT = 2, 3 or 4: 128 to 256 rows of x, 128 weight rows) and
+// walks K in chunks of 64, with two roles:
+// - eight compute waves, wave (wm, wn) = (wave % 4, wave / 4) multiplying its 16 MT x 64 block
+//   as MT x 4 16x16x32 MFMA tiles, two k-steps per chunk, from LDS only;
+// - eight loader waves, which load each chunk's x and packed weights three chunks ahead into
+//   registers (three sets in turn), then write x into LDS and dequantise the weights into it,
+//   w = round(fma(s, q, b)) in f32 then to bf16 / f16 (the rounding of MLX's dequantise,
+//   parity unpinned as to one rounding or two). The scales and biases of all of K are staged
+//   in LDS by the compute waves while the first chunks are in flight (2-byte loads of them per
+//   chunk each fetch a cache line: with 256 tiles of 192 rows, K = 4096, 62 us against 58);
+//   where they do not fit beside the buffers or are not 8-byte aligned, the loaders load them
+//   per chunk.
 // Two LDS buffers: the loaders fill chunk c + 1's while the compute waves multiply chunk
 // c's, one barrier per chunk. The loaders issue every load on every path (a chunk past the
-// end loads at offsets past the ranges: zeros, no memory access), so the compiler's waits
-// count exactly the chunk they need.
+// end loads at offsets past the ranges: zeros, no memory access), so the waits count exactly
+// the chunk they need.
 // LDS per buffer: x rows (128 bytes of a chunk each), then weight rows; the 16-byte units of
 // a row are swizzled, unit u at u ^ ((row >> 1) & 7), so that the 16 rows an MFMA operand
 // read touches at one unit land on 16 different bank groups (rows are 128 bytes: two per
@@ -661,9 +665,18 @@ int32_t launch_qmv_rows(hipStream_t st, const QmmArgs& a, int mx, const QmvPlan&
 // of tiles, consecutive workgroups (which the dispatcher spreads over the eight XCDs) take
 // the same place in different regions, so each XCD works through one region and its L2
 // holds that region's x rows and weight rows.
-constexpr int kDqBM = 256, kDqBN = 128, kDqKC = 64, kDqCompute = 8, kDqLoaders = 8;
-constexpr uint32_t kDqXBytes = kDqBM * 128, kDqBuf = kDqXBytes + kDqBN * 128;
-constexpr uint32_t kDqLds = 2 * kDqBuf;  // 96 KB: one workgroup per CU
+// Measured (8 bits, group 64, K = 4096, M = 1531): N = 6144 106 us (384 tiles of 192 rows, two
+// rounds) against 127 with 288 of 256 rows, N = 4096 58 against 65. A chunk costs 0.63, 0.70
+// and 0.84 us at MT = 2, 3, 4, of which only 0.21 to 0.43 are MFMA. Four compute waves of 32 MT
+// x 64 that read each operand one k-step ahead of its products (three buffers, four loader
+// waves) took 0.05 to 0.12 us more per chunk.
+constexpr int kDqBN = 128, kDqKC = 64, kDqCompute = 8, kDqLoaders = 8;
+template <int MT>
+struct Dq {
+  static constexpr int kBM = 64 * MT;
+  static constexpr uint32_t kXBytes = kBM * 128, kBuf = kXBytes + kDqBN * 128;
+  static constexpr uint32_t kLds = 2 * kBuf;  // 96, 80 or 64 KB
+};
 
 struct DqPlan {
   int mtiles, ntiles;
@@ -691,8 +704,10 @@ __device__ __forceinline__ uint32_t ld16u(u32x4 rs, uint32_t off) {
   return v;
 }
 
-template <int BITS, int GS, bool F16>
+template <int BITS, int GS, bool F16, int MT, bool kStaged>
 __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kernel(QmmArgs a, DqPlan p) {
+  constexpr int kDqBM = Dq<MT>::kBM;
+  constexpr uint32_t kDqXBytes = Dq<MT>::kXBytes, kDqBuf = Dq<MT>::kBuf;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   int mt, nt;
   if (p.rm > 0) {
@@ -720,9 +735,9 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
     const u32x4 Bi = rsrc4(a.b + (int64_t)n0 * G2, rows_n * G2);
     // x: unit u = ll % 8 of rows ll / 8 + 64 i (one load instruction covers 8 whole rows)
     const uint32_t xu = ll & 7, xr0 = ll >> 3;
-    uint32_t x_off[4];
+    uint32_t x_off[MT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < MT; ++i) {
       const uint32_t row = xr0 + 64 * i;
       x_off[i] = row < (uint32_t)rows_m ? row * xrow + 16 * xu : kOffRow;
     }
@@ -733,7 +748,7 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
     const bool w_in = wr_row < (uint32_t)rows_n;
     typedef uint32_t wv_t __attribute__((ext_vector_type(kWq)));
     struct Regs {
-      u32x4 x[4];
+      u32x4 x[MT];
       wv_t w;
       uint32_t s, b;
     };
@@ -741,29 +756,53 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
       const bool real = c < NC;
       const uint32_t cc = real ? (uint32_t)c : 0u, no = real ? 0u : kOffRow;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) r.x[i] = ld128(Xr, (x_off[i] | no) + cc * (2 * kDqKC));
+      for (int i = 0; i < MT; ++i) r.x[i] = ld128(Xr, (x_off[i] | no) + cc * (2 * kDqKC));
       const uint32_t k0 = cc * kDqKC + 16 * wh;
       const uint32_t wo = (w_in ? wr_row * wrow + k0 * BITS / 8 : kOffRow) | no;
       if constexpr (kWq == 2) r.w = ld64(W, wo);
       else r.w = ld128(W, wo);
-      const uint32_t so = (w_in ? wr_row * G2 + 2 * (k0 / GS) : kOffRow) | no;
-      r.s = ld16u(S, so);
-      r.b = ld16u(Bi, so);
+      if constexpr (!kStaged) {
+        const uint32_t so = (w_in ? wr_row * G2 + 2 * (k0 / GS) : kOffRow) | no;
+        r.s = ld16u(S, so);
+        r.b = ld16u(Bi, so);
+      }
     };
-    // loads per chunk: 4 of x, 1 of weights, 2 of scales and biases; staging a set waits
-    // for it with the two later sets' loads still in flight
+    // loads per chunk: MT of x, 1 of weights and, unless they are staged, 2 of scales and
+    // biases; staging a set waits for it with the two later sets' loads still in flight
     auto wait_set = [&](Regs& r) __attribute__((always_inline)) {
-      asm volatile("s_waitcnt vmcnt(14)"
-                   : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[2]), "+v"(r.x[3]), "+v"(r.w), "+v"(r.s), "+v"(r.b)
-                   :
-                   : "memory");
+      if constexpr (kStaged) {
+        if constexpr (MT == 4)
+          asm volatile("s_waitcnt vmcnt(10)" : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[2]), "+v"(r.x[MT - 1]), "+v"(r.w) : : "memory");
+        else if constexpr (MT == 3)
+          asm volatile("s_waitcnt vmcnt(8)" : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[MT - 1]), "+v"(r.w) : : "memory");
+        else
+          asm volatile("s_waitcnt vmcnt(6)" : "+v"(r.x[0]), "+v"(r.x[MT - 1]), "+v"(r.w) : : "memory");
+      } else {
+        if constexpr (MT == 4)
+          asm volatile("s_waitcnt vmcnt(14)" : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[2]), "+v"(r.x[MT - 1]), "+v"(r.w), "+v"(r.s), "+v"(r.b) : : "memory");
+        else if constexpr (MT == 3)
+          asm volatile("s_waitcnt vmcnt(12)" : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[MT - 1]), "+v"(r.w), "+v"(r.s), "+v"(r.b) : : "memory");
+        else
+          asm volatile("s_waitcnt vmcnt(10)" : "+v"(r.x[0]), "+v"(r.x[MT - 1]), "+v"(r.w), "+v"(r.s), "+v"(r.b) : : "memory");
+      }
     };
-    auto stage = [&](Regs& r, int buf) __attribute__((always_inline)) {
+    const uint32_t* const pairs = reinterpret_cast<const uint32_t*>(smem + 2 * kDqBuf) + wr_row * group_stride(a.G);
+    auto stage = [&](Regs& r, int c) __attribute__((always_inline)) {
+      const int buf = c & 1;
       wait_set(r);
       uint8_t* const xb = smem + (uint32_t)buf * kDqBuf;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(xb + 16 * dq_unit(xr0 + 64 * i, xu)) = r.x[i];
-      const float sc = act_to_f32<F16>(r.s), bc = act_to_f32<F16>(r.b);
+      for (int i = 0; i < MT; ++i) *reinterpret_cast<u32x4*>(xb + 16 * dq_unit(xr0 + 64 * i, xu)) = r.x[i];
+      uint32_t sw, bw;
+      if constexpr (kStaged) {
+        const uint32_t sb = pairs[((uint32_t)c * kDqKC + 16 * wh) / GS];
+        sw = sb & 0xffffu;
+        bw = sb >> 16;
+      } else {
+        sw = r.s;
+        bw = r.b;
+      }
+      const float sc = act_to_f32<F16>(sw), bc = act_to_f32<F16>(bw);
       uint8_t* const wb = xb + kDqXBytes;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {  // unit 2 wh + u: k 8 u .. 8 u + 7 of the quarter
@@ -779,19 +818,20 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
     load(0, r0);
     load(1, r1);
     load(2, r2);
+    if constexpr (kStaged) __syncthreads();  // the scales
     stage(r0, 0);
     __syncthreads();
     for (int c = 0; c < NC;) {
       load(c + 3, r0);
-      if (c + 1 < NC) stage(r1, (c + 1) & 1);
+      if (c + 1 < NC) stage(r1, c + 1);
       __syncthreads();
       if (++c >= NC) break;
       load(c + 3, r1);
-      if (c + 1 < NC) stage(r2, (c + 1) & 1);
+      if (c + 1 < NC) stage(r2, c + 1);
       __syncthreads();
       if (++c >= NC) break;
       load(c + 3, r2);
-      if (c + 1 < NC) stage(r0, (c + 1) & 1);
+      if (c + 1 < NC) stage(r0, c + 1);
       __syncthreads();
       ++c;
     }
@@ -802,11 +842,32 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
   // ---- compute
   const int wm = wave & 3, wn = wave >> 2;
   const uint32_t r16 = (uint32_t)lane & 15, j = (uint32_t)lane >> 4;
-  f32x4 acc[4][4];
+  f32x4 acc[MT][4];
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
+  for (int rt = 0; rt < MT; ++rt)
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (kStaged) {
+    // scales and biases of the 128 weight rows into LDS for the loaders, as {scale, bias}
+    // pairs, while these have their first chunks in flight
+    const uint32_t G = (uint32_t)a.G, stride = group_stride(G);
+    const auto S = rsrc(a.s + (int64_t)n0 * G * 2, rows_n * G * 2);
+    const auto Bi = rsrc(a.b + (int64_t)n0 * G * 2, rows_n * G * 2);
+    uint32_t* const pairs = reinterpret_cast<uint32_t*>(smem + 2 * kDqBuf);
+    // a lane takes four groups of a row, a wave `per` rows at a time
+    const uint32_t pieces = G / 4, sh = pieces >= 64 ? 6u : pieces <= 1 ? 0u : 32u - __builtin_clz(pieces - 1);
+    const uint32_t per = 64u >> sh;
+    for (uint32_t row = wave * per + (lane >> sh); row < (uint32_t)kDqBN; row += kDqCompute * per)
+      for (uint32_t g = 4 * (lane & ((1u << sh) - 1)); g < G; g += 256) {
+        const uint32_t off = row < (uint32_t)rows_n ? (row * G + g) * 2 : kOffRow;
+        const u32x2 sv = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(S, off, 0, 0));
+        const u32x2 bv = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(Bi, off, 0, 0));
+        *reinterpret_cast<u32x4*>(pairs + row * stride + g) =
+            u32x4{pair(sv[0], bv[0], kSelLo), pair(sv[0], bv[0], kSelHi), pair(sv[1], bv[1], kSelLo),
+                  pair(sv[1], bv[1], kSelHi)};
+      }
+    __syncthreads();
+  }
   __syncthreads();  // chunk 0 staged
   for (int c = 0; c < NC; ++c) {
     const uint8_t* const xb = smem + (uint32_t)(c & 1) * kDqBuf;
@@ -814,37 +875,46 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       const uint32_t u = 4 * ks + j;
-      u32x4 A[4], B[4];
+      u32x4 A[MT], B[4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        A[t] = *reinterpret_cast<const u32x4*>(xb + 16 * dq_unit(64 * wm + 16 * t + r16, u));
-        B[t] = *reinterpret_cast<const u32x4*>(wb + 16 * dq_unit(64 * wn + 16 * t + r16, u));
-      }
+      for (int t = 0; t < 4; ++t) B[t] = *reinterpret_cast<const u32x4*>(wb + 16 * dq_unit(64 * wn + 16 * t + r16, u));
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt)
+      for (int t = 0; t < MT; ++t)
+        A[t] = *reinterpret_cast<const u32x4*>(xb + 16 * dq_unit(16 * MT * wm + 16 * t + r16, u));
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = mma<F16>(A[rt], B[ct], acc[rt][ct]);
+      for (int rt = 0; rt < MT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = mma<F16>(B[ct], A[rt], acc[rt][ct]);
     }
     __syncthreads();
   }
 
-  // lane (r16, j) of tile (rt, ct) holds rows 4j .. 4j + 3 of column r16
+  // (weights, x) products: lane (r16, j) of tile (rt, ct) holds columns 4 j .. 4 j + 3 of row
+  // r16
+  const bool wide = (((uintptr_t)a.y | (uint64_t)a.ldy * 2) & 7) == 0;
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
+  for (int rt = 0; rt < MT; ++rt)
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct)
+    for (int ct = 0; ct < 4; ++ct) {
+      const int m = 16 * MT * wm + 16 * rt + (int)r16, n = 64 * wn + 16 * ct + 4 * (int)j;
+      if (m >= rows_m || n >= rows_n) continue;
+      uint16_t* const y = reinterpret_cast<uint16_t*>(a.y) + (int64_t)(m0 + m) * a.ldy + n0 + n;
+      const f32x4 v = acc[rt][ct];
+      if (wide && n + 4 <= rows_n) {
+        *reinterpret_cast<u32x2*>(y) = u32x2{pack_act2<F16>(v[0], v[1]), pack_act2<F16>(v[2], v[3])};
+      } else {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int m = 64 * wm + 16 * rt + 4 * (int)j + q, n = 64 * wn + 16 * ct + (int)r16;
-        if (m < rows_m && n < rows_n)
-          reinterpret_cast<uint16_t*>(a.y)[(int64_t)(m0 + m) * a.ldy + n0 + n] = f32_to_act<F16>(acc[rt][ct][q]);
+        for (int q = 0; q < 4; ++q)
+          if (n + q < rows_n) y[q] = f32_to_act<F16>(v[q]);
       }
+    }
 }
 
 // Plan of the dequantising GEMM: K a multiple of the chunk and of the group, x within one
 // buffer range per tile. Regions: 2 x 4, 4 x 2, 1 x 8 or 8 x 1 whole tile rows and columns,
 // the one with the least bytes per region, when the grid divides into them.
-bool plan_dq(int M, int N, int K, int gs, int bits, int64_t ldx, DqPlan* p) {
+bool plan_dq(int M, int N, int K, int gs, int bits, int64_t ldx, int mt, DqPlan* p) {
+  const int kDqBM = 64 * mt;
   if (K % kDqKC || K % gs || (int64_t)kDqBM * ldx * 2 + (int64_t)K * 2 >= ((int64_t)1 << 31)) return false;
   p->mtiles = (M + kDqBM - 1) / kDqBM;
   p->ntiles = (N + kDqBN - 1) / kDqBN;
@@ -865,16 +935,24 @@ bool plan_dq(int M, int N, int K, int gs, int bits, int64_t ldx, DqPlan* p) {
   return true;
 }
 
-template <int BITS, int GS, bool F16>
-int32_t launch_dq(hipStream_t st, const QmmArgs& a, const DqPlan& p) {
+template <int BITS, int GS, bool F16, int MT, bool kStaged>
+int32_t launch_dq_t(hipStream_t st, const QmmArgs& a, const DqPlan& p, uint32_t lds) {
   static std::atomic<uint64_t> lds_set{0};  // this instantiation's LDS above 64 KB, per device
-  const int32_t rc = allow_lds_once((const void*)qgemm_dq_kernel<BITS, GS, F16>, kDqLds, &lds_set,
+  const int32_t rc = allow_lds_once((const void*)qgemm_dq_kernel<BITS, GS, F16, MT, kStaged>, kQmvMaxLds, &lds_set,
                                     "quantized_matmul: LDS attribute");
   if (rc) return rc;
-  hipLaunchKernelGGL((qgemm_dq_kernel<BITS, GS, F16>), dim3((unsigned)(p.mtiles * p.ntiles)),
-                     dim3(64 * (kDqCompute + kDqLoaders)),
-                     kDqLds, st, a, p);
+  hipLaunchKernelGGL((qgemm_dq_kernel<BITS, GS, F16, MT, kStaged>), dim3((unsigned)(p.mtiles * p.ntiles)),
+                     dim3(64 * (kDqCompute + kDqLoaders)), lds, st, a, p);
   return check_hip(hipGetLastError(), "quantized_matmul launch");
+}
+
+template <int BITS, int GS, bool F16, int MT>
+int32_t launch_dq(hipStream_t st, const QmmArgs& a, const DqPlan& p) {
+  // scales through LDS: four groups per 8-byte load, all of K's pairs beside the buffers
+  const uint64_t staged = Dq<MT>::kLds + (uint64_t)kDqBN * group_stride((uint32_t)a.G) * 4;
+  if (a.G % 4 == 0 && (((uintptr_t)a.s | (uintptr_t)a.b) & 7) == 0 && staged <= kQmvMaxLds)
+    return launch_dq_t<BITS, GS, F16, MT, true>(st, a, p, (uint32_t)staged);
+  return launch_dq_t<BITS, GS, F16, MT, false>(st, a, p, Dq<MT>::kLds);
 }
 
 // ---------------------------------------------------------------- one row of x (M = 1)
@@ -1048,7 +1126,11 @@ int32_t launch_t(hipStream_t st, QmmArgs a) {
     const KsPlan kp = plan_ks(a, BITS, cus);
     if (kp.mt > 0) return launch_qgemm_ks(st, a, kp, GS, BITS, F16);
     DqPlan dp;
-    if (plan_dq(a.M, a.N, a.K, GS, BITS, a.ldx, &dp)) return launch_dq<BITS, GS, F16>(st, a, dp);
+    const int mt = dq_row_tiles(a.M, a.N, a.K, cus);
+    if (plan_dq(a.M, a.N, a.K, GS, BITS, a.ldx, mt, &dp))
+      return mt == 4   ? launch_dq<BITS, GS, F16, 4>(st, a, dp)
+             : mt == 3 ? launch_dq<BITS, GS, F16, 3>(st, a, dp)
+                       : launch_dq<BITS, GS, F16, 2>(st, a, dp);
   }
   const int mr = a.M <= 16 ? 1 : 2;
   a.mtiles = (a.M + 16 * mr - 1) / (16 * mr);

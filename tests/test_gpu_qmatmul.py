@@ -221,6 +221,30 @@ def test_qmatmul_ksplit_decode_rows(ema, ora, M, N, K, gs, bits, dtype):
     assert torch.all(wide[:, :1] == 7.0) and torch.all(wide[:, N + 1:] == 7.0)
 
 
+@pytest.mark.parametrize("M,N,K,gs,bits,dtype", [
+    # tiles of 128, 192 and 256 rows of the dequantising GEMM (chosen by the rounds on 256 CUs),
+    # ragged in both directions, scales staged in LDS or loaded per chunk (K / gs odd)
+    (1020, 4093, 128, 32, 4, "bf16"),   # 256 tiles of 128 rows
+    (1000, 4096, 192, 64, 8, "f16"),    # the same, three groups: loaded per chunk
+    (1530, 4090, 256, 32, 8, "bf16"),   # 256 tiles of 192 rows
+    (1531, 4096, 192, 64, 4, "f16"),
+    (2040, 4091, 128, 32, 4, "f16"),    # 256 tiles of 256 rows
+    (2047, 4096, 64, 64, 8, "bf16"),    # one chunk
+])
+def test_qmatmul_dequantising_tiles(ema, ora, M, N, K, gs, bits, dtype):
+    import torch
+
+    say(f"qmatmul dequantising tiles M={M} N={N} K={K} gs={gs} bits={bits} {dtype}")
+    d, h = make(ora, M + N + K, M, N, K, gs, bits, dtype)
+    y = ema.quantized_matmul(*d, group_size=gs, bits=bits)
+    check(ora, y, h, gs, bits, f"M={M}", dtype)
+    wide = torch.full((M, N + 3), 7.0, dtype=y.dtype, device="cuda")
+    ema.quantized_matmul(*d, group_size=gs, bits=bits, out=wide[:, 1:N + 1])
+    torch.cuda.synchronize()
+    assert torch.equal(wide[:, 1:N + 1].contiguous().view(torch.int16), y.view(torch.int16))
+    assert torch.all(wide[:, :1] == 7.0) and torch.all(wide[:, N + 1:] == 7.0)
+
+
 @pytest.mark.parametrize("M", [1, 32, 256])
 def test_qmatmul_graph_replay(ema, ora, M):
     # captured in a HIP graph and replayed several times with eager work between the

@@ -15,7 +15,8 @@
 // Halving the key range halves the longest causal work item, and workgroups are
 // dispatched heaviest first, so the short ones fill in behind the long ones. With two or
 // more query blocks per CU, each workgroup owns a heavy and a light block of one head and
-// runs them as one block stream per group (prefill_kernel<*, true>, described there).
+// runs them as one block stream per group (prefill_kernel<*, true>, described there). Few
+// query rows (a chat turn) run in prefill_few_kernel, 32 rows per workgroup.
 //
 // Both contractions run on MFMA 32x32x16 (bf16 in, f32 accumulate), in the transposed
 // form that keeps the softmax lane-local:
@@ -748,6 +749,224 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 }
 
+// ---------------------------------------------------------------- few query rows
+// A chat turn over a long history: at 157 rows and 32 heads prefill_kernel has 64 workgroups
+// of 128 rows, a quarter of the chip, and each walks all keys in 25 block steps. Here a
+// workgroup owns 32 query rows of one head, and its eight waves split the keys: wave w takes
+// the 32-key tiles w, w + 8, ..., all 32 rows, with its own K and V slot in LDS, and no
+// barrier until the eight (o, m, l) states of a row meet at the end. The products, the
+// scaling and rounding of Q, the bf16 rounding of P and the row sums over rounded P are those
+// of prefill_kernel; the running max moves per tile.
+// Each wave's K and V tiles come by LDS-DMA of whole rows. K of the next tile is requested
+// once QK has read the slot, V once PV has: K loads ride under softmax and PV, V loads under
+// the next QK and softmax, and the other wave of the SIMD fills the rest. Past its last tile a
+// wave requests offsets outside every range (zeros, no memory access), so that each wait
+// counts exactly the eight loads of the other tensor.
+constexpr int kFewM = 32, kFewWaves = 8, kFewTile = 32;
+constexpr int kFewSlot = kFewTile * kD * 2;                        // one K or V tile: 8 KB
+constexpr int kFewLds = kFewWaves * 2 * kFewSlot + kFewWaves * kFewM * 8;  // slots, then (m, l) per wave and row
+
+template <bool kRot>
+__global__ __launch_bounds__(64 * kFewWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_few_kernel(
+    PrefillArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the heads and row tiles of one (sequence, kv head) on one XCD (workgroups go round the
+  // eight XCDs), the last rows, which see the most keys, first
+  const int nq = a.nqb, per = a.G * nq;
+  const int l8 = blockIdx.x >> 3;
+  const int kvg = l8 / per * 8 + (int)(blockIdx.x & 7);
+  if (kvg >= a.B * a.Hkv) return;
+  const int b = kvg / a.Hkv, kh = kvg % a.Hkv;
+  const int inner = l8 % per;
+  const int row0 = (nq - 1 - inner / a.G) * kFewM, h = kh * a.G + inner % a.G;
+
+  int q_off = a.q_off[b];
+  q_off = q_off < 0 ? 0 : q_off;
+  int key_base = 0;  // absolute position of key index 0 (rotating cache)
+  if (kRot) {
+    key_base = q_off + a.T - a.cap;
+    key_base = key_base < 0 ? 0 : key_base;
+    q_off -= key_base;
+  }
+  int kv_len = q_off + a.T;
+  kv_len = kv_len > a.cap ? a.cap : kv_len;
+  const bool causal = a.flags & EMA_PREFILL_CAUSAL;
+  int kv_begin = (a.flags & EMA_PREFILL_CHUNK_ONLY) ? q_off : 0;
+  kv_begin = kv_begin > kv_len ? kv_len : kv_begin;
+  int end = kv_len;  // keys of the workgroup's last row
+  if (causal && q_off + row0 + kFewM < end) end = q_off + row0 + kFewM;
+  const int t_begin = kv_begin / kFewTile, t_end = (end + kFewTile - 1) / kFewTile;
+
+  const int hh = lane >> 5, r4 = lane >> 4, p16 = lane & 15;
+  const uint32_t row_bytes = (uint32_t)a.sp * 2, ring_bytes = (uint32_t)a.cap * row_bytes;
+  const uint32_t kv_bytes = (uint32_t)kv_len * row_bytes;
+  const u32x4 k_rsrc = buffer_rsrc(a.k + (int64_t)b * a.sb + (int64_t)kh * a.sh, kv_bytes);
+  const u32x4 v_rsrc = buffer_rsrc(a.v + (int64_t)b * a.sb + (int64_t)kh * a.sh, kv_bytes);
+  uint16_t* const Kt = lds + wave * kFewSlot;  // (elements: one wave's K and V tiles)
+  uint16_t* const Vt = Kt + kFewTile * kD;
+  const uint32_t kdst = (uint32_t)(uintptr_t)(lds_void*)Kt, vdst = (uint32_t)(uintptr_t)(lds_void*)Vt;
+  // source chunk of position p16 in row 4 i + r4: p16 ^ (row & 15) for K, p16 ^ 4 (row & 3) for V
+  uint32_t kchunk[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) kchunk[i] = (uint32_t)(p16 ^ (4 * i + r4)) * 16;
+  const uint32_t vchunk = (uint32_t)(p16 ^ (4 * r4)) * 16;
+  // eight instructions of 4 rows each; rows outside [kv_begin, kv_len) arrive as zeros
+  auto load_tile = [&](u32x4 r, bool k, int t) __attribute__((always_inline)) {
+    const int c0 = t * kFewTile;
+    const int ring = kRot ? (key_base + c0) % a.cap : c0;  // cache row of the tile's first key
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int at = 4 * i + r4;
+      int row = ring + at;
+      if (kRot && row >= a.cap) row -= a.cap;
+      uint32_t off = (uint32_t)row * row_bytes + (k ? kchunk[i & 3] : vchunk);
+      if (t >= t_end || c0 + at < kv_begin || c0 + at >= kv_len) off = kNoRow;
+      dma16<0>(r, off, (k ? kdst : vdst) + 1024 * i);
+    }
+  };
+
+  // Q^T as B operand: step s covers dims 16 s + 8 hh .. + 7 of row lane & 31
+  bf16x8 qop[8];
+  {
+    const int qr = row0 + (lane & 31) < a.T ? row0 + (lane & 31) : a.T - 1;
+    const u32x4* const qp = (const u32x4*)(a.q + (((int64_t)b * a.Hq + h) * a.T + qr) * kD) + hh;
+    u32x4 raw[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) raw[s] = qp[2 * s];
+    load_tile(k_rsrc, true, t_begin + wave);
+    load_tile(v_rsrc, false, t_begin + wave);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      u32x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        w[e] = pack_bf16x2(bf16_lo(raw[s][e]) * a.qk_scale, bf16_hi(raw[s][e]) * a.qk_scale);
+      qop[s] = as_bf16x8(w);
+    }
+  }
+  // operand reads, as in prefill_kernel: K row lane & 31, column chunk 2 s + hh at chunk
+  // (2 s + hh) ^ (lane & 15); V^T by the transposing read
+  const uint16_t* const kp = Kt + (lane & 31) * kD + 8 * (hh ^ (lane & 1));
+  const int k_x = 16 * ((lane & 15) >> 1);
+  const int grp = lane >> 4, s16 = lane & 15;
+  const int tr_row = 4 * (grp >> 1) + (s16 >> 2);
+  int v_col[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) v_col[dt] = tr_row * kD + 16 * (grp & 1) + 4 * (s16 & 3) + 32 * (dt ^ (s16 >> 2));
+
+  float m = -INFINITY, l = 0.f;  // of row lane & 31; l over this lane's half of the keys
+  f32x16 o[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
+  const int last_key = causal && q_off + row0 + (lane & 31) < kv_len - 1 ? q_off + row0 + (lane & 31) : kv_len - 1;
+
+  for (int t = t_begin + wave; t < t_end; t += kFewWaves) {
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // K of this tile
+    f32x16 sc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sc[i] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) sc = mfma32(as_bf16x8(*(const u32x4*)(kp + (k_x ^ (16 * s)))), qop[s], sc);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot has been read
+    load_tile(k_rsrc, true, t + kFewWaves);
+    // key of score i: 32 t + (i % 4) + 8 (i / 4) + 4 hh
+    const int kb = t * kFewTile + 4 * hh;
+    if (t * kFewTile < kv_begin || t * kFewTile + kFewTile > kv_len ||
+        (causal && t * kFewTile + kFewTile - 1 > q_off + row0)) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int key = kb + (i & 3) + 8 * (i >> 2);
+        sc[i] = key <= last_key && key >= kv_begin ? sc[i] : -INFINITY;
+      }
+    }
+    float mx = sc[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, sc[i]);
+    mx = fmaxf(wave_max_xor(mx, 32), m);
+    if (__any(mx > m)) {  // some row's max grew: rescale what was accumulated
+      const float alpha = mx == m ? 1.f : __builtin_amdgcn_exp2f(m - mx);
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
+      m = mx;
+    }
+    const float base = m == -INFINITY ? 0.f : m;
+    u32x4 pw[2];
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 8 * st + 2 * e;
+        pw[st][e] = pack_bf16x2(__builtin_amdgcn_exp2f(sc[i] - base), __builtin_amdgcn_exp2f(sc[i + 1] - base));
+        l = dot2_bf16(pw[st][e], 0x3F803F80u, l);
+      }
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // V of this tile
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        const uint16_t* const p0 = Vt + 16 * st * kD + v_col[dt];
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p0);
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + 8 * kD));
+        typedef short s16x8 __attribute__((ext_vector_type(8)));
+        const s16x8 av = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        o[dt] = mfma32(__builtin_bit_cast(bf16x8, av), as_bf16x8(pw[st]), o[dt]);
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    load_tile(v_rsrc, false, t + kFewWaves);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (zeros past the range)
+
+  // the states meet: o of wave w in its own slots, [row][dim / 4] f32x4 with chunk d4 of row r
+  // at d4 ^ r, (m, l) behind the slots
+  f32x4* const os = (f32x4*)Kt;
+  float2* const ml = (float2*)((uint8_t*)lds + kFewWaves * 2 * kFewSlot);
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const int d4 = 8 * dt + 2 * i4 + hh, r = lane & 31;
+      os[r * 32 + (d4 ^ r)] = f32x4{o[dt][4 * i4], o[dt][4 * i4 + 1], o[dt][4 * i4 + 2], o[dt][4 * i4 + 3]};
+    }
+  l += __shfl_xor(l, 32, 64);
+  if (lane < 32) ml[wave * kFewM + lane] = float2{m, l};
+  __syncthreads();
+  const int r = tid >> 4, c8 = tid & 15;  // row, 8 dims
+  float mt = -INFINITY;
+  float2 s[kFewWaves];
+#pragma unroll
+  for (int w = 0; w < kFewWaves; ++w) {
+    s[w] = ml[w * kFewM + r];
+    mt = fmaxf(mt, s[w].x);
+  }
+  f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
+  float lt = 0.f;
+#pragma unroll
+  for (int w = 0; w < kFewWaves; ++w) {
+    const float f = s[w].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s[w].x - mt);
+    const f32x4* const ow = (const f32x4*)(lds + w * kFewSlot) + r * 32;
+    lt += s[w].y * f;
+    acc0 += ow[(2 * c8) ^ r] * f;
+    acc1 += ow[(2 * c8 + 1) ^ r] * f;
+  }
+  const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+  if (row0 + r < a.T)
+    *(u32x4*)(a.out + (((int64_t)b * a.T + row0 + r) * a.Hq + h) * kD + 8 * c8) =
+        u32x4{pack_bf16x2(acc0[0] * inv, acc0[1] * inv), pack_bf16x2(acc0[2] * inv, acc0[3] * inv),
+              pack_bf16x2(acc1[0] * inv, acc1[1] * inv), pack_bf16x2(acc1[2] * inv, acc1[3] * inv)};
+}
+
+// Whether the items (32 query rows of one head) go to prefill_few_kernel: when they are one
+// round of workgroups on the CUs, whatever the history (its length is on the device). Measured,
+// us here / prefill_kernel, 32 heads: 157 rows after 3000 27 / 42, 16 after 12000 70 / 125, 128
+// from the start 7.9 / 9.7, 256 (256 items) 9.5 / 11.7; past one round 300 rows after 6000 (320
+// items) 82 / 75, 512 from the start 16.8 / 14.5.
+bool prefill_few(int64_t items, int cus) { return items <= cus; }
+
 }  // namespace
 
 int32_t launch_prefill(hipStream_t s, const void* q, const ema_kvcache_desc& c,
@@ -785,13 +1004,28 @@ int32_t launch_prefill(hipStream_t s, const void* q, const ema_kvcache_desc& c,
   a.cap = c.capacity;
   a.nqb = (T + kBM - 1) / kBM;
   a.flags = flags;
-  // pair the query blocks when there are at least two workgroups' worth per CU
   const int cus = device_cus();
+  const bool rot = c.flags & EMA_KV_ROTATING;
+  const int few_rows = (T + kFewM - 1) / kFewM;
+  if (prefill_few((int64_t)few_rows * Hq * c.batch, cus)) {
+    static std::atomic<uint64_t> few_set[2];
+    const void* fk = rot ? (const void*)prefill_few_kernel<true> : (const void*)prefill_few_kernel<false>;
+    const int32_t rc = allow_lds_once(fk, kFewLds, &few_set[rot ? 1 : 0], "ema_prefill_attention: LDS attribute");
+    if (rc) return rc;
+    a.nqb = few_rows;
+    a.paired = 0;
+    const int64_t blocks = (int64_t)((c.batch * c.n_kv_heads + 7) / 8) * 8 * a.G * few_rows;
+    if (rot)
+      hipLaunchKernelGGL(prefill_few_kernel<true>, dim3((unsigned)blocks), dim3(64 * kFewWaves), kFewLds, s, a);
+    else
+      hipLaunchKernelGGL(prefill_few_kernel<false>, dim3((unsigned)blocks), dim3(64 * kFewWaves), kFewLds, s, a);
+    return check_hip(hipGetLastError(), "ema_prefill_attention launch");
+  }
+  // pair the query blocks when there are at least two workgroups' worth per CU
   const int64_t items = (int64_t)a.nqb * Hq * c.batch;
   a.paired = a.nqb >= 2 && items >= 2 * (int64_t)cus;
   const int64_t blocks = prefill_grid(c.batch, Hq, a.nqb, a.paired);
   if (blocks > 0x7fffffff) return set_error(EMA_ERR_SHAPE, "ema_prefill_attention: grid too large");
-  const bool rot = c.flags & EMA_KV_ROTATING;
   if (rot && a.paired)
     hipLaunchKernelGGL((prefill_kernel<true, true>), dim3((unsigned)blocks), dim3(kThreads), kLdsBytes, s, a);
   else if (rot)

@@ -435,6 +435,24 @@ def test_prefill_small(ema, ora, T, q_off, causal, chunk, G):
     assert_close(got, ref, f"prefill T={T}")
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,T,q_off,causal,chunk", [
+    # 32 query rows per workgroup (at most 256 of them): fewer key tiles than waves, whole and
+    # partial tiles and row blocks, kv heads not a multiple of the XCDs, the largest grid
+    (3, 6, 3, 31, [0, 1, 33], True, False),
+    (3, 6, 3, 32, [224, 225, 256], True, False),
+    (1, 12, 3, 33, [991], True, False),
+    (2, 8, 1, 64, [959, 32], False, False),
+    (2, 8, 2, 65, [31, 500], True, True),
+    (5, 10, 5, 97, [0, 63, 64, 65, 300], False, True),
+    (2, 32, 8, 128, [700, 0], True, False),
+    (1, 32, 8, 157, [850], True, False),
+])
+def test_prefill_few_rows(ema, ora, B, Hq, Hkv, T, q_off, causal, chunk):
+    say(f"prefill few rows B={B} Hq={Hq} Hkv={Hkv} T={T} q_off={q_off} causal={causal} chunk={chunk}")
+    got, ref = _prefill_case(ema, ora, B, Hq, Hkv, 128, 1024, T, q_off, causal, chunk, seed=350 + T + B)
+    assert_close(got, ref, "prefill few rows")
+
+
 @pytest.mark.parametrize("causal,chunk", [(True, False), (False, False), (True, True)])
 def test_prefill_xcd_grid_mapping(ema, ora, causal, chunk):
     """batch x kv heads a multiple of 8 (the XCD-grouped grid order), ragged offsets."""

@@ -153,6 +153,26 @@ def test_rotating_prefill_window(ema, ora, q_off, T, W, chunk):
     assert_close(host(out), ref, f"prefill W={W}")
 
 
+@pytest.mark.parametrize("T", [96, 300])
+def test_rotating_prefill_few_rows_and_unpaired(ema, ora, T):
+    """Ring rows with 32 query rows per workgroup (T 96: 192 of them, a ring whose wrap falls
+    inside a 32-key tile) and with 128, unpaired (T 300: 640 items of 32)."""
+    import torch
+
+    B, Hq, Hkv, D, W = 4, 16, 4, 128, 1000
+    qo = np.asarray((0, 950, 1500, 2113), np.int32)
+    L = qo + T
+    say(f"rotating prefill T={T} W={W} q_off={qo.tolist()}")
+    big_k = ora.normal_bf16((B, Hkv, int(L.max()), D), seed=81)
+    big_v = ora.normal_bf16((B, Hkv, int(L.max()), D), seed=82)
+    q = ora.normal_bf16((B, Hq, T, D), seed=83)
+    cache = ring_cache(ema, ring_from(ora, big_k, L, W), ring_from(ora, big_v, L, W))
+    out = ema.prefill_attention(dev(q), cache, dev(qo), causal=True)
+    torch.cuda.synchronize()
+    ref = ora.sdpa(q, big_k, big_v, L, scale_of(D), True, kv_begin=np.maximum(L - W, 0))
+    assert_close(host(out), ref, f"rotating prefill T={T}")
+
+
 @pytest.mark.parametrize("q_off,chunk", [
     ((0, 300, 1500, 2100), False),  # one sequence without a wrap, three wrapping
     ((100, 1200, 40, 2500), True),  # chunk-only keys

@@ -626,9 +626,12 @@ KsPlan plan_ks(const QmmArgs& a, int bits, int cus) {
 // one against 10.4; N = 9216, two rounds either way, 17.3 with one against 19.5). Below K =
 // 2048 (fewer than two units per wave) the staged kernel of qmatmul.hip is the faster one:
 // K = 1024, N = 2048 3.6 against 3.9 us at 8 rows, 5.0 against 6.1 at 32; K = 2048 4.6
-// against 4.1 and 7.6 against 6.5.
-KsPlan plan_qmv_ks(const QmmArgs& a, int cus) {
-  if (a.K < 2 * kKsWaves * kUnit || !ks_fits(a)) return KsPlan{0, 0};
+// against 4.1 and 7.6 against 6.5. With 8 bits the line for up to 16 rows is K = 4096: at M = 2,
+// nine layers of K = 2048 to N = 4096 and 2048 take 87 us there and 97 here; K = N = 4096 7.9
+// us against 7.6 at 2 rows and 8.5 against 7.6 at 8.
+KsPlan plan_qmv_ks(const QmmArgs& a, int bits, int cus) {
+  const int min_k = (bits == 8 && a.M <= 16 ? 4 : 2) * kKsWaves * kUnit;
+  if (a.K < min_k || !ks_fits(a)) return KsPlan{0, 0};
   const int t1 = (a.N + 15) / 16, t2 = (a.N + 31) / 32;
   return KsPlan{a.M > 16 ? 2 : 1, t1 <= cus || t2 > cus ? 1 : 2};
 }

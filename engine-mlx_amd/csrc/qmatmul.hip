@@ -14,7 +14,7 @@
 // Two regimes, as in MLX, whose quantized matmul takes vector kernels for a few rows of x
 // and, for many, kernels that dequantise weight tiles into the activation type first:
 // - up to 32 rows (and the streaming fallback): exact products, below, and qgemm_ks.hip from
-//   K = 2048 on;
+//   K = 2048 on (8 bits and up to 16 rows: from K = 4096 on);
 // - more than 32 rows with K a multiple of 64: qgemm_dq_kernel, and the K-split kernel of
 //   qgemm_ks.hip where small tiles fill the chip better, on weights dequantised into bf16 /
 //   f16 (one rounding each).
@@ -1104,7 +1104,7 @@ int32_t launch_t(hipStream_t st, QmmArgs a) {
   const int cus = device_cus();
   if (a.M == 1 && gemv1_fits(a.G, a.K)) return launch_gemv1<BITS, GS, F16>(st, a, cus);
   if (a.M <= 32) {
-    const KsPlan kp = plan_qmv_ks(a, cus);
+    const KsPlan kp = plan_qmv_ks(a, BITS, cus);
     if (kp.mt > 0) return launch_qmv_ks(st, a, kp, GS, BITS, F16);
     const int mx = qmv_rows(a.M);
     const QmvPlan p = plan_qmv(a.N, a.K, GS, BITS, mx, cus);

@@ -40,7 +40,7 @@ struct KsPlan {
 KsPlan plan_ks(const QmmArgs& a, int bits, int cus);
 int32_t launch_qgemm_ks(hipStream_t st, const QmmArgs& a, const KsPlan& p, int gs, int bits, bool f16);
 // The same for the exact products of up to 32 rows.
-KsPlan plan_qmv_ks(const QmmArgs& a, int cus);
+KsPlan plan_qmv_ks(const QmmArgs& a, int bits, int cus);
 int32_t launch_qmv_ks(hipStream_t st, const QmmArgs& a, const KsPlan& p, int gs, int bits, bool f16);
 
 namespace {

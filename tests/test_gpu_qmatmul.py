@@ -194,11 +194,12 @@ def test_qmatmul_ksplit_tiles(ema, ora, M, N, K, gs, bits, dtype):
 
 
 @pytest.mark.parametrize("M,N,K,gs,bits,dtype", [
-    # exact products split over K (K >= 2048): 8, 16 and 32 rows, one and two column tiles,
+    # exact products split over K (K >= 2048; 8 bits and up to 16 rows K >= 4096): 8, 16 and 32 rows, one and two column tiles,
     # ragged columns, units that do not divide among the eight waves
     (2, 70, 2048, 64, 4, "bf16"),
     (8, 33, 2176, 32, 4, "f16"),        # 17 units
-    (9, 100, 2048, 128, 8, "bf16"),
+    (9, 100, 4096, 128, 8, "bf16"),
+    (9, 100, 3968, 128, 8, "bf16"),     # 8 bits, up to 16 rows, below K = 4096: the staged kernel
     (16, 4099, 2048, 64, 4, "bf16"),    # two column tiles, ragged
     (17, 48, 2560, 64, 8, "f16"),       # 20 units
     (31, 4110, 2304, 32, 4, "bf16"),    # two column tiles, 18 units

@@ -600,10 +600,12 @@ bool ks_fits(const QmmArgs& a) {
 // = 2048 and 4096, in units of 25 ns: a workgroup takes 140 and, per turn of its eight waves
 // over a unit each, 4 + 16 per row tile + 18 per column tile (qgemm_dq_kernel: dq_cost; K =
 // 4096, N = 4096: 33 us here against 45 at 300 rows, 45 against 45 at 520, 58 against 46 at
-// 700).
+// 700). The column tiles of an XCD all read all of x, so it has to stay in its 4 MB L2: K = 2048,
+// N = 1024 21.5 us here against 24 at 1200 rows (4.7 MB), 25.1 against 24.5 at 1531 (6 MB) and
+// 39.9 against 23.8 at 2048 (8 MB).
 KsPlan plan_ks(const QmmArgs& a, int bits, int cus) {
   KsPlan best{0, 0};
-  if (!ks_fits(a)) return best;
+  if (!ks_fits(a) || (int64_t)a.M * a.K * 2 > (5 << 20)) return best;
   auto rounds = [&](int rows, int cols) {
     return (((int64_t)a.M + rows - 1) / rows * (((int64_t)a.N + cols - 1) / cols) + cus - 1) / cus;
   };

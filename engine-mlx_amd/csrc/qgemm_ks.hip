@@ -14,9 +14,10 @@
 // of x): a quarter wave of a buffer load touches two lines. Straight loads in MFMA layout
 // (lane = row + 16 * piece) touch 16 lines per quarter wave and took 54 to 67 cycles per
 // load, whatever their size. The registers then pass through a few KB of LDS that belong to
-// the wave (write by rows, read in MFMA layout; no barrier, a wave's LDS operations are in
-// order) while the next unit's loads are in flight behind them. Scales and biases are staged
-// once per workgroup as {scale, bias} pairs.
+// the wave (write by rows, read in MFMA layout; wave_lds_fence in between, which emits nothing:
+// a wave's LDS operations execute in order, and the fence has the compiler keep that order)
+// while the next unit's loads are in flight behind them. Scales and biases are staged once per
+// workgroup as {scale, bias} pairs.
 // MFMA step i (32 k) needs fields 8 j .. 8 j + 7 of the step in lane row j:
 // - 4 bits: dword i of lane row j holds fields 32 j + 8 i ..; a 4 x 4 transpose between lane
 //   rows and registers (v_permlane16_swap, v_permlane32_swap: four instructions per 16
@@ -173,8 +174,8 @@ __global__ __launch_bounds__(64 * kKsWaves) void qgemm_ks_kernel(QmmArgs a, int 
 
   // The wave's LDS scratch: slots of 16 rows x 128 bytes, 16-byte piece p of row r at
   // p ^ ((r >> 1) & 7); 16 rows x 64 bytes for 4-bit weights, piece p at p ^ (r >> 2) (both
-  // free of bank conflicts). A wave's LDS operations execute in order, so a slot is reused
-  // without a barrier.
+  // free of bank conflicts). A slot is written again four exchanges later, behind the fences of
+  // the three in between.
   uint8_t* const slots = smem + slot_off + (uint32_t)wave * (kSlots * kSlot);
   const uint32_t wr8 = lane >> 3, wp8 = lane & 7, wr4 = lane >> 2;
   const uint32_t put8 = wr8 * 128 + 16 * (wp8 ^ (wr8 >> 1));  // rows 0 .. 7; rows 8 .. 15 below
@@ -196,6 +197,7 @@ __global__ __launch_bounds__(64 * kKsWaves) void qgemm_ks_kernel(QmmArgs a, int 
       uint8_t* const sl = next_slot();
       if constexpr (BITS == 4) {
         *reinterpret_cast<u32x4*>(sl + put4) = wr[t][0];
+        wave_lds_fence();
         const u32x4 v = *reinterpret_cast<const u32x4*>(sl + c * 64 + 16 * (j ^ (c >> 2)));
         uint32_t d0 = v[0], d1 = v[1], d2 = v[2], d3 = v[3];
         swap16(d0, d1);
@@ -209,6 +211,7 @@ __global__ __launch_bounds__(64 * kKsWaves) void qgemm_ks_kernel(QmmArgs a, int 
       } else {
         *reinterpret_cast<u32x4*>(sl + put8) = wr[t][0];
         *reinterpret_cast<u32x4*>(sl + put8h) = wr[t][kWL - 1];
+        wave_lds_fence();
 #pragma unroll
         for (int e = 0; e < kWL; ++e) {
           const u32x4 v = *reinterpret_cast<const u32x4*>(sl + c * 128 + 16 * ((4 * e + j) ^ (c >> 1)));
@@ -223,34 +226,38 @@ __global__ __launch_bounds__(64 * kKsWaves) void qgemm_ks_kernel(QmmArgs a, int 
       }
     }
     if constexpr (refill.value) load_w(next);
+    // x by row tile, each multiplied right behind its reads: the fences keep the exchanges in
+    // this order, and all row tiles of a line read first took 20 registers too many at 5 x 3
+    // (4 bits, N = 6144, K = 4096, 157 rows: 24.1 us against 18.4)
 #pragma unroll
     for (int ln = 0; ln < 2; ++ln) {
-      u32x4 xv[2][MT];
+      u32x4 wv[2][NT];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int st = 2 * ln + h;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const uint32_t sb = gl[16 * t * gs4 + cur * (kUnit / GS) + st * 32 / GS];
+          const float s = act_to_f32<F16>(sb & 0xffffu), b = act_to_f32<F16>(sb >> 16);
+          if constexpr (BITS == 4) wv[h][t] = dequant8<BITS, F16>(wd[t][st], 0u, s, b);
+          else wv[h][t] = dequant8<BITS, F16>(wd[t][2 * st], wd[t][2 * st + 1], s, b);
+        }
+      }
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
         uint8_t* const sl = next_slot();
         *reinterpret_cast<u32x4*>(sl + put8) = xr[ln][t][0];
         *reinterpret_cast<u32x4*>(sl + put8h) = xr[ln][t][1];
+        wave_lds_fence();
+        u32x4 xv[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          xv[h][t] = *reinterpret_cast<const u32x4*>(sl + c * 128 + 16 * ((4 * h + xj) ^ (c >> 1)));
+          xv[h] = *reinterpret_cast<const u32x4*>(sl + c * 128 + 16 * ((4 * h + xj) ^ (c >> 1)));
         if constexpr (refill.value) load_x(next, ln, t);
-      }
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int st = 2 * ln + h;
-        u32x4 wv[NT];
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const uint32_t sb = gl[16 * t * gs4 + cur * (kUnit / GS) + st * 32 / GS];
-          const float s = act_to_f32<F16>(sb & 0xffffu), b = act_to_f32<F16>(sb >> 16);
-          if constexpr (BITS == 4) wv[t] = dequant8<BITS, F16>(wd[t][st], 0u, s, b);
-          else wv[t] = dequant8<BITS, F16>(wd[t][2 * st], wd[t][2 * st + 1], s, b);
-        }
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-          for (int n = 0; n < NT; ++n) acc[n][m] = mma<F16>(wv[n], xv[h][m], acc[n][m]);
+          for (int n = 0; n < NT; ++n) acc[n][t] = mma<F16>(wv[h][n], xv[h], acc[n][t]);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -418,6 +425,7 @@ __global__ __launch_bounds__(64 * kKsWaves) void qmv_ks_kernel(QmmArgs a, uint32
       uint8_t* const sl = next_slot();
       if constexpr (BITS == 4) {
         *reinterpret_cast<u32x4*>(sl + put4) = wr[ws][t][0];
+        wave_lds_fence();
         const u32x4 v = *reinterpret_cast<const u32x4*>(sl + c * 64 + 16 * (j ^ (c >> 2)));
         uint32_t d0 = v[0], d1 = v[1], d2 = v[2], d3 = v[3];
         swap16(d0, d1);
@@ -431,6 +439,7 @@ __global__ __launch_bounds__(64 * kKsWaves) void qmv_ks_kernel(QmmArgs a, uint32
       } else {
         *reinterpret_cast<u32x4*>(sl + put8) = wr[ws][t][0];
         *reinterpret_cast<u32x4*>(sl + put8h) = wr[ws][t][kWL - 1];
+        wave_lds_fence();
 #pragma unroll
         for (int e = 0; e < kWL; ++e) {
           const u32x4 v = *reinterpret_cast<const u32x4*>(sl + c * 128 + 16 * ((4 * e + j) ^ (c >> 1)));
@@ -444,6 +453,13 @@ __global__ __launch_bounds__(64 * kKsWaves) void qmv_ks_kernel(QmmArgs a, uint32
         }
       }
     }
+    // the unit's pairs ahead of x's fences, which they could not pass (8 bits, group 32, N = K =
+    // 5120, 16 rows: 14.0 us when read at the end of a group, 13.2 here)
+    uint32_t sb[NT][kUnit / GS];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int g = 0; g < kUnit / GS; ++g) sb[n][g] = gl[16 * n * gs4 + cur * (kUnit / GS) + g];
 #pragma unroll
     for (int ln = 0; ln < 2; ++ln) {
       u32x4 xv[2][MT];
@@ -453,6 +469,7 @@ __global__ __launch_bounds__(64 * kKsWaves) void qmv_ks_kernel(QmmArgs a, uint32
         *reinterpret_cast<u32x4*>(sl + put8) = xr[xs][ln][t][0];
         // rows 8 .. 15 of an 8-row call hold what the slot held: rows that are not stored
         if constexpr (H == 2) *reinterpret_cast<u32x4*>(sl + put8h) = xr[xs][ln][t][H - 1];
+        wave_lds_fence();
 #pragma unroll
         for (int h = 0; h < 2; ++h)
           xv[h][t] = *reinterpret_cast<const u32x4*>(sl + c * 128 + 16 * ((4 * h + xj) ^ (c >> 1)));
@@ -482,8 +499,8 @@ __global__ __launch_bounds__(64 * kKsWaves) void qmv_ks_kernel(QmmArgs a, uint32
         if ((st + 1) * 32 % GS == 0) {
 #pragma unroll
           for (int n = 0; n < NT; ++n) {
-            const uint32_t sb = gl[16 * n * gs4 + cur * (kUnit / GS) + st * 32 / GS];
-            const float sc = act_to_f32<F16>(sb & 0xffffu), bc = act_to_f32<F16>(sb >> 16) - F::kOff * sc;
+            const uint32_t p = sb[n][st * 32 / GS];
+            const float sc = act_to_f32<F16>(p & 0xffffu), bc = act_to_f32<F16>(p >> 16) - F::kOff * sc;
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll

@@ -54,6 +54,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
 
+// Between a wave's LDS writes and its reads of what its other lanes wrote: the hardware runs a
+// wave's LDS operations in order, and this has the compiler keep that order, which it may not
+// otherwise when it can tell a lane's own write and read apart. No instructions.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <bool F16>
 __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
   if constexpr (F16)

@@ -61,6 +61,34 @@ EMA_HD int64_t prefill_grid(int B, int Hq, int nqb, int paired) {
   return (int64_t)(paired ? (nqb + 1) / 2 : nqb) * B * Hq;
 }
 
+// Few query rows (a chat turn): items of kFewM query rows of one head, eight waves over the
+// keys of each. The kernel runs one workgroup per CU, and each XCD gets an equal share of the
+// items: a contiguous piece of them in the order of their (sequence, kv head) group, so that
+// the workgroups that read the same K and V meet on one XCD, two where a group straddles the
+// cut. Measured, us (whole groups per XCD / items round the XCDs where the groups do not
+// divide over them / here): 32 heads on 1 kv head, 256 rows 49.8 / 9.6 / 9.6; on 4, 157 rows
+// after 3000 48.4 / 27.2 / 27.0; 5 sequences of 10 on 5, 129 rows after 3000 47.3 / 50.0 / 28.8.
+// It takes the calls whose items are one round of workgroups, whatever the history (its length
+// is on the device). Measured, us here / prefill_kernel, 32 heads: 157 rows after 3000 26.6 /
+// 42.1, 16 after 12000 70.9 / 125, 128 from the start 7.9 / 9.7, 256 (256 items) 9.6 / 12.0;
+// past one round 300 rows after 6000 (320 items) 82 / 75, 512 from the start 16.8 / 14.5.
+constexpr int kFewM = 32;
+EMA_HD int prefill_few_blocks(int T) { return (T + kFewM - 1) / kFewM; }
+EMA_HD bool prefill_few(int B, int Hq, int T, int cus) { return (int64_t)prefill_few_blocks(T) * Hq * B <= cus; }
+// Item of workgroup x of `grid` = prefill_grid(B, Hkv * G, nq, 0), nq = prefill_few_blocks(T).
+EMA_HD PrefillItem prefill_few_item(int x, int grid, int Hkv, int G, int nq) {
+  const int xcd = x % kSchedXcds, extra = grid % kSchedXcds;
+  const int rank = xcd * (grid / kSchedXcds) + (xcd < extra ? xcd : extra) + x / kSchedXcds;
+  const int grp = rank / (G * nq), inner = rank % (G * nq);
+  PrefillItem it;
+  it.qb_first = nq - 1 - inner / G;
+  it.qb_second = it.qb_first;
+  it.b = grp / Hkv;
+  it.kh = grp % Hkv;
+  it.h = it.kh * G + inner % G;
+  return it;
+}
+
 // Block streams of a prefill workgroup's two wave groups. A query block attends the
 // 64-key blocks [blk_begin, blk_begin + n) of its key range; the heavy block has nblk_h
 // of them, the light block of a pair nblk_l <= nblk_h (0 without a light block: a single

@@ -762,7 +762,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 // the next QK and softmax, and the other wave of the SIMD fills the rest. Past its last tile a
 // wave requests offsets outside every range (zeros, no memory access), so that each wait
 // counts exactly the eight loads of the other tensor.
-constexpr int kFewM = 32, kFewWaves = 8, kFewTile = 32;
+constexpr int kFewWaves = 8, kFewTile = 32;
 constexpr int kFewSlot = kFewTile * kD * 2;                        // one K or V tile: 8 KB
 constexpr int kFewLds = kFewWaves * 2 * kFewSlot + kFewWaves * kFewM * 8;  // slots, then (m, l) per wave and row
 
@@ -772,15 +772,8 @@ __global__ __launch_bounds__(64 * kFewWaves) __attribute__((amdgpu_waves_per_eu(
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // the heads and row tiles of one (sequence, kv head) on one XCD (workgroups go round the
-  // eight XCDs), the last rows, which see the most keys, first
-  const int nq = a.nqb, per = a.G * nq;
-  const int l8 = blockIdx.x >> 3;
-  const int kvg = l8 / per * 8 + (int)(blockIdx.x & 7);
-  if (kvg >= a.B * a.Hkv) return;
-  const int b = kvg / a.Hkv, kh = kvg % a.Hkv;
-  const int inner = l8 % per;
-  const int row0 = (nq - 1 - inner / a.G) * kFewM, h = kh * a.G + inner % a.G;
+  const PrefillItem item = prefill_few_item((int)blockIdx.x, (int)gridDim.x, a.Hkv, a.G, a.nqb);
+  const int b = item.b, kh = item.kh, h = item.h, row0 = item.qb_first * kFewM;
 
   int q_off = a.q_off[b];
   q_off = q_off < 0 ? 0 : q_off;
@@ -800,7 +793,7 @@ __global__ __launch_bounds__(64 * kFewWaves) __attribute__((amdgpu_waves_per_eu(
   const int t_begin = kv_begin / kFewTile, t_end = (end + kFewTile - 1) / kFewTile;
 
   const int hh = lane >> 5, r4 = lane >> 4, p16 = lane & 15;
-  const uint32_t row_bytes = (uint32_t)a.sp * 2, ring_bytes = (uint32_t)a.cap * row_bytes;
+  const uint32_t row_bytes = (uint32_t)a.sp * 2;
   const uint32_t kv_bytes = (uint32_t)kv_len * row_bytes;
   const u32x4 k_rsrc = buffer_rsrc(a.k + (int64_t)b * a.sb + (int64_t)kh * a.sh, kv_bytes);
   const u32x4 v_rsrc = buffer_rsrc(a.v + (int64_t)b * a.sb + (int64_t)kh * a.sh, kv_bytes);
@@ -960,13 +953,6 @@ __global__ __launch_bounds__(64 * kFewWaves) __attribute__((amdgpu_waves_per_eu(
               pack_bf16x2(acc1[0] * inv, acc1[1] * inv), pack_bf16x2(acc1[2] * inv, acc1[3] * inv)};
 }
 
-// Whether the items (32 query rows of one head) go to prefill_few_kernel: when they are one
-// round of workgroups on the CUs, whatever the history (its length is on the device). Measured,
-// us here / prefill_kernel, 32 heads: 157 rows after 3000 27 / 42, 16 after 12000 70 / 125, 128
-// from the start 7.9 / 9.7, 256 (256 items) 9.5 / 11.7; past one round 300 rows after 6000 (320
-// items) 82 / 75, 512 from the start 16.8 / 14.5.
-bool prefill_few(int64_t items, int cus) { return items <= cus; }
-
 }  // namespace
 
 int32_t launch_prefill(hipStream_t s, const void* q, const ema_kvcache_desc& c,
@@ -1006,15 +992,14 @@ int32_t launch_prefill(hipStream_t s, const void* q, const ema_kvcache_desc& c,
   a.flags = flags;
   const int cus = device_cus();
   const bool rot = c.flags & EMA_KV_ROTATING;
-  const int few_rows = (T + kFewM - 1) / kFewM;
-  if (prefill_few((int64_t)few_rows * Hq * c.batch, cus)) {
+  if (prefill_few(c.batch, Hq, T, cus)) {
     static std::atomic<uint64_t> few_set[2];
     const void* fk = rot ? (const void*)prefill_few_kernel<true> : (const void*)prefill_few_kernel<false>;
     const int32_t rc = allow_lds_once(fk, kFewLds, &few_set[rot ? 1 : 0], "ema_prefill_attention: LDS attribute");
     if (rc) return rc;
-    a.nqb = few_rows;
+    a.nqb = prefill_few_blocks(T);
     a.paired = 0;
-    const int64_t blocks = (int64_t)((c.batch * c.n_kv_heads + 7) / 8) * 8 * a.G * few_rows;
+    const int64_t blocks = prefill_grid(c.batch, Hq, a.nqb, 0);
     if (rot)
       hipLaunchKernelGGL(prefill_few_kernel<true>, dim3((unsigned)blocks), dim3(64 * kFewWaves), kFewLds, s, a);
     else

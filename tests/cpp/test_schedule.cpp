@@ -4,7 +4,8 @@
 //    paired or not, with and without the XCD grouping; the heavy block of a pair runs
 //    first; with the XCD grouping every item of a (sequence, kv head) group lands on the
 //    group's XCD; ranks run heaviest first; inside a workgroup the two wave groups' block
-//    streams see each (row set, key block) once and stay balanced;
+//    streams see each (row set, key block) once and stay balanced; calls of few query rows
+//    are one round of workgroups, spread evenly over the XCDs;
 //  - decode split: the worker slices tile [0, total) exactly once, split_worker_of
 //    inverts split_begin, the merge's slot range [w0, w1] of every segment is exactly the
 //    set of slices that intersect it, and the partial-state slots (w + segment) of split
@@ -83,6 +84,48 @@ static void test_prefill() {
     for (int paired = 0; paired < 2; ++paired) prefill_case(s[0], s[1], s[2], s[3], paired);
   std::printf("prefill schedule: %zu shapes x {unpaired, paired}: every (b, h, qb) exactly once\n",
               sizeof(shapes) / sizeof(shapes[0]));
+}
+
+// Calls of few query rows: every (sequence, head, row block) once, and, since a workgroup
+// holds a CU to itself, no more on an XCD than it has CUs (a second round) nor more than an
+// even spread gives it.
+static void test_prefill_few() {
+  const int cus = 256;
+  int cases = 0;
+  for (int B = 1; B <= 12; ++B)
+    for (int Hkv = 1; Hkv <= 16; ++Hkv)
+      for (int G : {1, 2, 3, 4, 8, 16, 32})
+        for (int T : {1, 16, 31, 32, 33, 65, 96, 129, 157, 200, 256, 300, 512, 1000, 4096}) {
+          if (!prefill_few(B, Hkv * G, T, cus)) continue;
+          const int nq = prefill_few_blocks(T);
+          const int64_t grid = prefill_grid(B, Hkv * G, nq, 0);
+          CHECK(grid == (int64_t)B * Hkv * G * nq, "a workgroup without an item");
+          std::set<std::vector<int>> seen;
+          int on_xcd[kSchedXcds] = {};
+          std::vector<std::set<int>> xcds(B * Hkv);
+          for (int64_t x = 0; x < grid; ++x) {
+            const PrefillItem it = prefill_few_item((int)x, (int)grid, Hkv, G, nq);
+            CHECK(it.b >= 0 && it.b < B && it.h / G == it.kh && it.kh >= 0 && it.kh < Hkv, "x=%lld outside", (long long)x);
+            CHECK(it.qb_first >= 0 && it.qb_first < nq && it.qb_second == it.qb_first, "x=%lld rows", (long long)x);
+            CHECK(seen.insert({it.b, it.h, it.qb_first}).second, "item run twice (x=%lld)", (long long)x);
+            ++on_xcd[x % kSchedXcds];
+            xcds[it.b * Hkv + it.kh].insert((int)(x % kSchedXcds));
+          }
+          CHECK((int64_t)seen.size() == grid, "items missed");
+          for (int n : on_xcd)
+            CHECK(n <= cus / kSchedXcds && n <= (grid + kSchedXcds - 1) / kSchedXcds,
+                  "B=%d Hkv=%d G=%d T=%d: %d of %lld workgroups on one XCD", B, Hkv, G, T, n, (long long)grid);
+          // a group meets as many XCDs as its items need, one more where it straddles a cut
+          const int least = (int)(grid / kSchedXcds);
+          for (const auto& g : xcds)
+            CHECK((int)g.size() <= (least ? (G * nq + least - 1) / least + 1 : kSchedXcds), "B=%d Hkv=%d G=%d T=%d: a group on %zu XCDs",
+                  B, Hkv, G, T, g.size());
+          ++cases;
+        }
+  // the largest calls taken, and the first not taken
+  CHECK(prefill_few(1, 32, 256, cus) && !prefill_few(1, 32, 257, cus), "32 heads");
+  CHECK(prefill_few(1, 8, 1024, cus) && !prefill_few(2, 8, 1024, cus), "8 heads");
+  std::printf("few-row prefill: %d calls, each item once, one round of workgroups\n", cases);
 }
 
 // Decode split for tile counts nb[s] per segment s (segments in sequence-major order).
@@ -277,6 +320,7 @@ static void test_decode_slots() {
 int main() {
   test_prefill();
   test_prefill_streams();
+  test_prefill_few();
   test_decode();
   test_decode_slots();
   std::printf("%d checks passed\n", g_checks);

@@ -446,6 +446,12 @@ def test_prefill_small(ema, ora, T, q_off, causal, chunk, G):
     (5, 10, 5, 97, [0, 63, 64, 65, 300], False, True),
     (2, 32, 8, 128, [700, 0], True, False),
     (1, 32, 8, 157, [850], True, False),
+    # 4, 2 and 1 kv heads (spread over the whole chip) at the largest grid and below it
+    (1, 32, 4, 256, [512], True, False),
+    (1, 16, 2, 512, [301], True, False),
+    (1, 32, 1, 256, [0], False, False),
+    (1, 8, 1, 1000, [24], True, False),
+    (3, 16, 4, 157, [0, 700, 33], True, True),
 ])
 def test_prefill_few_rows(ema, ora, B, Hq, Hkv, T, q_off, causal, chunk):
     say(f"prefill few rows B={B} Hq={Hq} Hkv={Hkv} T={T} q_off={q_off} causal={causal} chunk={chunk}")

@@ -61,6 +61,13 @@ EMA_HD int64_t prefill_grid(int B, int Hq, int nqb, int paired) {
   return (int64_t)(paired ? (nqb + 1) / 2 : nqb) * B * Hq;
 }
 
+// Place of workgroup x of `grid` in an order of the work items of which each XCD takes an equal,
+// contiguous share (the first grid % 8 XCDs one more): neighbours in that order meet on one XCD.
+EMA_HD int xcd_rank(int x, int grid) {
+  const int xcd = x % kSchedXcds, extra = grid % kSchedXcds;
+  return xcd * (grid / kSchedXcds) + (xcd < extra ? xcd : extra) + x / kSchedXcds;
+}
+
 // Few query rows (a chat turn): items of kFewM query rows of one head, eight waves over the
 // keys of each. The kernel runs one workgroup per CU, and each XCD gets an equal share of the
 // items: a contiguous piece of them in the order of their (sequence, kv head) group, so that
@@ -77,8 +84,7 @@ EMA_HD int prefill_few_blocks(int T) { return (T + kFewM - 1) / kFewM; }
 EMA_HD bool prefill_few(int B, int Hq, int T, int cus) { return (int64_t)prefill_few_blocks(T) * Hq * B <= cus; }
 // Item of workgroup x of `grid` = prefill_grid(B, Hkv * G, nq, 0), nq = prefill_few_blocks(T).
 EMA_HD PrefillItem prefill_few_item(int x, int grid, int Hkv, int G, int nq) {
-  const int xcd = x % kSchedXcds, extra = grid % kSchedXcds;
-  const int rank = xcd * (grid / kSchedXcds) + (xcd < extra ? xcd : extra) + x / kSchedXcds;
+  const int rank = xcd_rank(x, grid);
   const int grp = rank / (G * nq), inner = rank % (G * nq);
   PrefillItem it;
   it.qb_first = nq - 1 - inner / G;
@@ -87,6 +93,18 @@ EMA_HD PrefillItem prefill_few_item(int x, int grid, int Hkv, int G, int nq) {
   it.kh = grp % Hkv;
   it.h = it.kh * G + inner % G;
   return it;
+}
+
+// ------------------------------------------------------------------ K-split projections
+// Tile of workgroup x of the K-split GEMM's grid of ntiles x mtiles: the row tiles of a column
+// tile side by side in xcd_rank's order, so that one XCD's L2 serves the re-reads of its weights
+// (two where it straddles a cut), and no XCD has more workgroups than an even share.
+struct KsTile {
+  int nt, mt;
+};
+EMA_HD KsTile ks_tile_of(int x, int grid, int mtiles) {
+  const int rank = xcd_rank(x, grid);
+  return KsTile{rank / mtiles, rank % mtiles};
 }
 
 // Block streams of a prefill workgroup's two wave groups. A query block attends the

@@ -32,6 +32,7 @@
 // byte written and read once) and MFMA, which add up rather than overlap; staging the next
 // line before the current one's MFMAs, or other wave priorities, changed nothing.
 #include "qmatmul_common.hpp"
+#include "ema_schedule.hpp"
 
 #include <type_traits>
 
@@ -99,15 +100,11 @@ struct GroupStage {
 };
 
 template <int BITS, int GS, bool F16, int MT, int NT>
-__global__ __launch_bounds__(64 * kKsWaves) void qgemm_ks_kernel(QmmArgs a, int ntiles, uint32_t slot_off) {
+__global__ __launch_bounds__(64 * kKsWaves) void qgemm_ks_kernel(QmmArgs a, uint32_t slot_off) {
   constexpr int kWL = BITS / 4;  // 16-byte weight loads per unit and column tile
-  constexpr int kRows = 16 * NT;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  // the row tiles of one column tile on one XCD (workgroups go round the eight XCDs), so its
-  // L2 serves the re-reads of their weights
-  const int l = blockIdx.x >> 3;
-  const int nt = (l / a.mtiles) * 8 + (int)(blockIdx.x & 7), mt = l % a.mtiles;
-  if (nt >= ntiles) return;
+  const KsTile tile = ks_tile_of((int)blockIdx.x, (int)gridDim.x, a.mtiles);
+  const int nt = tile.nt, mt = tile.mt;
   const int n0 = nt * 16 * NT, m0 = mt * 16 * MT;
   const int rows_n = min(16 * NT, a.N - n0), rows_m = min(16 * MT, a.M - m0);
   const int lane = threadIdx.x & 63;
@@ -139,7 +136,7 @@ __global__ __launch_bounds__(64 * kKsWaves) void qgemm_ks_kernel(QmmArgs a, int 
   const int units = a.K / kUnit;
   // units wave, wave + 8, ... of a walk of K that starts at another place in each workgroup
   const int count = (units - wave + kKsWaves - 1) / kKsWaves;
-  int u = (l * kKsWaves + wave) % units;
+  int u = ((nt / 8 * a.mtiles + mt) * kKsWaves + wave) % units;
 
   u32x4 xr[2][MT][2], wr[NT][kWL];  // x: [line of the unit][row tile][half of its rows]
   auto load_w = [&](int u) __attribute__((always_inline)) {
@@ -556,8 +553,8 @@ int32_t launch(hipStream_t st, const QmmArgs& a) {
   const uint32_t lds = used > kRed ? used : kRed;
   QmmArgs b = a;
   b.mtiles = (a.M + 16 * MT - 1) / (16 * MT);
-  hipLaunchKernelGGL((qgemm_ks_kernel<BITS, GS, F16, MT, NT>), dim3((unsigned)((ntiles + 7) / 8 * 8 * b.mtiles)),
-                     dim3(64 * kKsWaves), lds, st, b, ntiles, slot_off);
+  hipLaunchKernelGGL((qgemm_ks_kernel<BITS, GS, F16, MT, NT>), dim3((unsigned)(ntiles * b.mtiles)),
+                     dim3(64 * kKsWaves), lds, st, b, slot_off);
   return check_hip(hipGetLastError(), "quantized_matmul launch");
 }
 

@@ -6,6 +6,7 @@
 //    group's XCD; ranks run heaviest first; inside a workgroup the two wave groups' block
 //    streams see each (row set, key block) once and stay balanced; calls of few query rows
 //    are one round of workgroups, spread evenly over the XCDs;
+//  - K-split projections: every tile once, an even share of them on each XCD;
 //  - decode split: the worker slices tile [0, total) exactly once, split_worker_of
 //    inverts split_begin, the merge's slot range [w0, w1] of every segment is exactly the
 //    set of slices that intersect it, and the partial-state slots (w + segment) of split
@@ -126,6 +127,37 @@ static void test_prefill_few() {
   CHECK(prefill_few(1, 32, 256, cus) && !prefill_few(1, 32, 257, cus), "32 heads");
   CHECK(prefill_few(1, 8, 1024, cus) && !prefill_few(2, 8, 1024, cus), "8 heads");
   std::printf("few-row prefill: %d calls, each item once, one round of workgroups\n", cases);
+}
+
+// The K-split GEMM's grids: every tile once, an even share per XCD (so a grid of one workgroup
+// per CU is one round, as its plan counts), a column tile's row tiles on as few XCDs as hold them.
+static void test_ks_tiles() {
+  const int cus = 256;
+  int cases = 0;
+  for (int ntiles = 1; ntiles <= 130; ++ntiles)
+    for (int mtiles = 1; mtiles <= 24; ++mtiles) {
+      const int grid = ntiles * mtiles, least = grid / kSchedXcds;
+      std::vector<int> seen(grid, 0);
+      std::vector<std::set<int>> xcds(ntiles);
+      int on_xcd[kSchedXcds] = {};
+      for (int x = 0; x < grid; ++x) {
+        const KsTile t = ks_tile_of(x, grid, mtiles);
+        CHECK(t.nt >= 0 && t.nt < ntiles && t.mt >= 0 && t.mt < mtiles, "x=%d tile %d %d", x, t.nt, t.mt);
+        ++seen[t.nt * mtiles + t.mt];
+        ++on_xcd[x % kSchedXcds];
+        xcds[t.nt].insert(x % kSchedXcds);
+      }
+      for (int i = 0; i < grid; ++i) CHECK(seen[i] == 1, "%d x %d: tile %d run %d times", ntiles, mtiles, i, seen[i]);
+      for (int n : on_xcd) {
+        const int rounds = (n + cus / kSchedXcds - 1) / (cus / kSchedXcds);
+        CHECK(rounds <= (grid + cus - 1) / cus, "%d x %d: %d rounds on one XCD", ntiles, mtiles, rounds);
+      }
+      for (const auto& s : xcds)
+        CHECK((int)s.size() <= (least ? (mtiles + least - 1) / least + 1 : kSchedXcds), "%d x %d: a column tile on %zu XCDs",
+              ntiles, mtiles, s.size());
+      ++cases;
+    }
+  std::printf("K-split tiles: %d grids, each tile once, rounds as the plan counts them\n", cases);
 }
 
 // Decode split for tile counts nb[s] per segment s (segments in sequence-major order).
@@ -321,6 +353,7 @@ int main() {
   test_prefill();
   test_prefill_streams();
   test_prefill_few();
+  test_ks_tiles();
   test_decode();
   test_decode_slots();
   std::printf("%d checks passed\n", g_checks);

@@ -32,17 +32,14 @@
 // byte written and read once) and MFMA, which add up rather than overlap; staging the next
 // line before the current one's MFMAs, or other wave priorities, changed nothing.
 #include "qmatmul_common.hpp"
-#include "ema_schedule.hpp"
 
 #include <type_traits>
 
 namespace ema {
 namespace {
 
-constexpr int kKsWaves = 8;
-constexpr int kKsMaxLds = 160 * 1024;
-constexpr int kUnit = 128;            // k per unit
 constexpr uint32_t kSlots = 4, kSlot = 2048;
+static_assert(kKsWaves * kSlots * kSlot == kKsSlotBytes, "the plan counts these slots");
 
 __device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {
   const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
@@ -583,12 +580,6 @@ int32_t launch_tile_v(hipStream_t st, const QmmArgs& a, const KsPlan& p) {
                      : launch_v<BITS, GS, F16, 32, 2>(st, a);
 }
 
-// Tiles whose kernel fits the registers: 8-bit weights take twice the registers in flight,
-// and at 5 x 3 and 4 x 4 they spill.
-constexpr bool ks_tile(int bits, int mt, int nt) {
-  return mt >= 3 && mt <= 5 && nt >= 2 && nt <= 4 && mt + nt <= (bits == 4 ? 8 : 7);
-}
-
 template <int BITS, int GS, bool F16>
 int32_t launch_tile(hipStream_t st, const QmmArgs& a, const KsPlan& p) {
 #define EMA_KS(m, n) \
@@ -599,58 +590,7 @@ int32_t launch_tile(hipStream_t st, const QmmArgs& a, const KsPlan& p) {
   return set_error(EMA_ERR_UNSUPPORTED, "quantized_matmul: no kernel for tile %d x %d", p.mt, p.nt);
 }
 
-// Whole units, four groups' scales or biases per 8-byte load, the pairs of 64 rows and the
-// slots within the LDS, 32-bit offsets inside a tile of 80 rows.
-bool ks_fits(const QmmArgs& a) {
-  return a.K % kUnit == 0 && a.G % 4 == 0 && (((uintptr_t)a.s | (uintptr_t)a.b) & 7) == 0 &&
-         (a.G + 4) * 64 * 4 + kKsWaves * (int)(kSlots * kSlot) <= kKsMaxLds &&
-         80 * a.ldx * 2 + (int64_t)a.K * 2 < ((int64_t)1 << 31);
-}
-
 }  // namespace
-
-// The tile, or mt = 0 when qgemm_dq_kernel is the better kernel or this one does not apply.
-// One workgroup per CU at a time, so a call takes rounds * time of a workgroup; measured at K
-// = 2048 and 4096, in units of 25 ns: a workgroup takes 140 and, per turn of its eight waves
-// over a unit each, 4 + 16 per row tile + 18 per column tile (qgemm_dq_kernel: dq_cost; K =
-// 4096, N = 4096: 33 us here against 45 at 300 rows, 45 against 45 at 520, 58 against 46 at
-// 700). The column tiles of an XCD all read all of x, so it has to stay in its 4 MB L2: K = 2048,
-// N = 1024 21.5 us here against 24 at 1200 rows (4.7 MB), 25.1 against 24.5 at 1531 (6 MB) and
-// 39.9 against 23.8 at 2048 (8 MB).
-KsPlan plan_ks(const QmmArgs& a, int bits, int cus) {
-  KsPlan best{0, 0};
-  if (!ks_fits(a) || (int64_t)a.M * a.K * 2 > (5 << 20)) return best;
-  auto rounds = [&](int rows, int cols) {
-    return (((int64_t)a.M + rows - 1) / rows * (((int64_t)a.N + cols - 1) / cols) + cus - 1) / cus;
-  };
-  int64_t cost = dq_cost(a.M, a.N, a.K, dq_row_tiles(a.M, a.N, a.K, cus), cus);
-  const int64_t turns = (a.K / kUnit + kKsWaves - 1) / kKsWaves;
-  for (int mt = 3; mt <= 5; ++mt)
-    for (int nt = 2; nt <= 4; ++nt) {
-      if (!ks_tile(bits, mt, nt)) continue;
-      const int64_t c = rounds(16 * mt, 16 * nt) * (140 + turns * (4 + 16 * mt + 18 * nt));
-      if (c < cost) {
-        cost = c;
-        best = KsPlan{mt, nt};
-      }
-    }
-  return best;
-}
-
-// One column tile per workgroup while those fit the CUs in one round, else two while these
-// do (measured at M = 32, K = 4096: N = 6144 10.8 us with two against 12.1, N = 4096 8.6 with
-// one against 10.4; N = 9216, two rounds either way, 17.3 with one against 19.5). Below K =
-// 2048 (fewer than two units per wave) the staged kernel of qmatmul.hip is the faster one:
-// K = 1024, N = 2048 3.6 against 3.9 us at 8 rows, 5.0 against 6.1 at 32; K = 2048 4.6
-// against 4.1 and 7.6 against 6.5. With 8 bits the line for up to 16 rows is K = 4096: at M = 2,
-// nine layers of K = 2048 to N = 4096 and 2048 take 87 us there and 97 here; K = N = 4096 7.9
-// us against 7.6 at 2 rows and 8.5 against 7.6 at 8.
-KsPlan plan_qmv_ks(const QmmArgs& a, int bits, int cus) {
-  const int min_k = (bits == 8 && a.M <= 16 ? 4 : 2) * kKsWaves * kUnit;
-  if (a.K < min_k || !ks_fits(a)) return KsPlan{0, 0};
-  const int t1 = (a.N + 15) / 16, t2 = (a.N + 31) / 32;
-  return KsPlan{a.M > 16 ? 2 : 1, t1 <= cus || t2 > cus ? 1 : 2};
-}
 
 int32_t launch_qmv_ks(hipStream_t st, const QmmArgs& a, const KsPlan& p, int gs, int bits, bool f16) {
 #define EMA_KS(f) \

@@ -201,20 +201,6 @@ typedef __attribute__((address_space(3))) void lds_void;
 //            unit u of the row, then row % 8:  unit (rb, u, row % 8) <- row, bytes [16 u, +16)
 //   x slot   unit u of the chunk, then row r:  unit (u, r) <- x row r, chunk bytes [16 u, +16)
 //   scales   unit (g / 8, row) <- row, groups [g, g + 8); biases likewise
-constexpr uint32_t kQmvMaxLds = 160 * 1024;  // all of a gfx950 CU's LDS
-
-struct QmvPlan {
-  int NT, KCH, NC, NB;
-  uint32_t U;         // weight units per row (all of K)
-  uint32_t Uc;        // weight units per row per chunk
-  uint32_t rb_bytes;  // one row block plus padding
-  uint32_t x_off;     // first x slot
-  uint32_t x_slot;    // bytes per x slot
-  uint32_t nW, nX;    // DMA instructions per chunk (weights, x)
-  uint32_t nS;        // DMA instructions for all scales (and again for the biases)
-  uint32_t s_off, b_off, z_off, bytes;
-};
-
 // 0..31 outstanding vector-memory operations; larger counts wait for 31 (a longer wait).
 __device__ __forceinline__ void wait_vmcnt(uint32_t n) {
   switch (n) {
@@ -374,55 +360,6 @@ __global__ __launch_bounds__(64 * kMaxWaves) void qmv_kernel(QmmArgs a, QmvPlan 
 }
 
 
-// Plan of the staged kernel for M <= 32 rows, or NC = 0 when it does not apply: a chunk
-// is whole DMA blocks per weight row block (KCH * bits / 128 a multiple of 8) and whole
-// groups, K is a multiple of it, and K / gs is a multiple of 8 (each 16-byte scale load
-// ends inside its row).
-QmvPlan plan_qmv(int N, int K, int gs, int bits, int mx, int cus) {
-  QmvPlan none{};
-  none.NC = 0;
-  if ((K / gs) % 8 != 0) return none;
-  const int G = K / gs;
-  // two column tiles per workgroup only when 16-column tiles would outnumber the CUs (a
-  // second round of workgroups costs more than doubling each one's columns)
-  const int nt0 = mx >= 8 && (N + 15) / 16 > cus ? 2 : 1;
-  for (int nt = nt0; nt >= 1; --nt) {
-    const int rows = 16 * nt;
-    for (int kch = 1024; kch >= 128; kch /= 2) {
-      if (K % kch || kch % gs || (kch * bits / 128) % 8) continue;
-      if (nt == 2 && kch < 256) continue;  // measured: more chunks cost more than a second round
-      QmvPlan q{};
-      q.NT = nt;
-      q.KCH = kch;
-      q.NC = K / kch;
-      q.U = (uint32_t)K * bits / 128;
-      q.Uc = (uint32_t)kch * bits / 128;
-      q.rb_bytes = q.U * 128 + 128;
-      q.nW = (uint32_t)rows * q.Uc / 64;
-      q.nX = ((uint32_t)mx * kch / 8 + 63) / 64;
-      q.x_slot = 1024 * q.nX;
-      q.nS = ((uint32_t)rows * (G / 8) + 63) / 64;
-      q.x_off = ((2 * nt) * q.rb_bytes + 1023) & ~1023u;
-      const uint32_t fixed = q.x_off + 2 * 1024 * q.nS;
-      // all of x if it fits (then everything is in flight from the start), else the
-      // deepest ring that fits beside the weights
-      int nb = q.NC;
-      while (nb > 2 && fixed + 16 + nb * q.x_slot > kQmvMaxLds) --nb;
-      q.NB = nb;
-      q.s_off = q.x_off + nb * q.x_slot;
-      q.b_off = q.s_off + 1024 * q.nS;
-      q.z_off = q.b_off + 1024 * q.nS;  // 16 zero bytes read by rows of x past M
-      q.bytes = q.z_off + 16;
-      const uint32_t red = (uint32_t)kMaxWaves * (mx > 16 ? 2 : 1) * 1024;
-      if (q.bytes < red) q.bytes = red;
-      // the largest chunk that fits: fewer chunks, fewer barriers (measured faster at
-      // 32 rows than deeper rings of smaller chunks)
-      if (q.bytes <= kQmvMaxLds) return q;
-    }
-  }
-  return none;
-}
-
 // Variant for 16 or 32 rows of x: the weights, scales and biases are staged in LDS as in
 // qmv_kernel (all of K, one round of DMA and one barrier), but x does not pass through LDS:
 // each wave loads its own x straight into registers in MFMA layout, kXD groups ahead and
@@ -569,39 +506,6 @@ __global__ __launch_bounds__(64 * kMaxWaves) void qmvx_kernel(QmmArgs a, QmvPlan
   }
 }
 
-// Plan of qmvx_kernel: all weights and scales of 16 NT rows in LDS (x not staged).
-QmvPlan plan_qmvx(int N, int K, int gs, int bits, int cus) {
-  QmvPlan none{};
-  none.NC = 0;
-  if ((K / gs) % 8 != 0 || (K * bits / 128) % 8 != 0) return none;
-  const int G = K / gs;
-  const int nt0 = (N + 15) / 16 > cus ? 2 : 1;
-  for (int nt = nt0; nt >= 1; --nt) {
-    const int rows = 16 * nt;
-    QmvPlan q{};
-    q.NT = nt;
-    q.KCH = K;
-    q.NC = 1;
-    q.NB = 1;
-    q.U = (uint32_t)K * bits / 128;
-    q.Uc = q.U;
-    q.rb_bytes = q.U * 128 + 128;
-    q.nW = (uint32_t)rows * q.U / 64;
-    q.nX = 0;
-    q.x_slot = 0;
-    q.nS = ((uint32_t)rows * (G / 8) + 63) / 64;
-    q.x_off = ((2 * nt) * q.rb_bytes + 1023) & ~1023u;
-    q.s_off = q.x_off;
-    q.b_off = q.s_off + 1024 * q.nS;
-    q.z_off = q.b_off + 1024 * q.nS;
-    q.bytes = q.z_off + 16;
-    const uint32_t red = (uint32_t)kMaxWaves * 2 * 1024;
-    if (q.bytes < red) q.bytes = red;
-    if (q.bytes <= kQmvMaxLds) return q;
-  }
-  return none;
-}
-
 template <int BITS, int GS, bool F16, int MX, int NT>
 int32_t launch_qmvx(hipStream_t st, const QmmArgs& a, const QmvPlan& p) {
   static std::atomic<uint64_t> lds_set{0};  // this instantiation's LDS above 64 KB, per device
@@ -623,8 +527,6 @@ int32_t launch_qmv(hipStream_t st, const QmmArgs& a, const QmvPlan& p) {
                      dim3(64 * kMaxWaves), p.bytes, st, a, p);
   return check_hip(hipGetLastError(), "quantized_matmul launch");
 }
-
-int qmv_rows(int M) { return M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 8 ? 8 : M <= 16 ? 16 : 32; }
 
 template <int BITS, int GS, bool F16>
 int32_t launch_qmv_rows(hipStream_t st, const QmmArgs& a, int mx, const QmvPlan& p) {
@@ -670,17 +572,11 @@ int32_t launch_qmv_rows(hipStream_t st, const QmmArgs& a, int mx, const QmvPlan&
 // and 0.84 us at MT = 2, 3, 4, of which only 0.21 to 0.43 are MFMA. Four compute waves of 32 MT
 // x 64 that read each operand one k-step ahead of its products (three buffers, four loader
 // waves) took 0.05 to 0.12 us more per chunk.
-constexpr int kDqBN = 128, kDqKC = 64, kDqCompute = 8, kDqLoaders = 8;
 template <int MT>
 struct Dq {
   static constexpr int kBM = 64 * MT;
   static constexpr uint32_t kXBytes = kBM * 128, kBuf = kXBytes + kDqBN * 128;
   static constexpr uint32_t kLds = 2 * kBuf;  // 96, 80 or 64 KB
-};
-
-struct DqPlan {
-  int mtiles, ntiles;
-  int rm, rn;  // tile rows / columns per region (regions: mtiles / rm x ntiles / rn = 8), or 0
 };
 
 __device__ __forceinline__ uint32_t dq_unit(uint32_t row, uint32_t u) { return row * 8 + (u ^ ((row >> 1) & 7)); }
@@ -910,31 +806,6 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
     }
 }
 
-// Plan of the dequantising GEMM: K a multiple of the chunk and of the group, x within one
-// buffer range per tile. Regions: 2 x 4, 4 x 2, 1 x 8 or 8 x 1 whole tile rows and columns,
-// the one with the least bytes per region, when the grid divides into them.
-bool plan_dq(int M, int N, int K, int gs, int bits, int64_t ldx, int mt, DqPlan* p) {
-  const int kDqBM = 64 * mt;
-  if (K % kDqKC || K % gs || (int64_t)kDqBM * ldx * 2 + (int64_t)K * 2 >= ((int64_t)1 << 31)) return false;
-  p->mtiles = (M + kDqBM - 1) / kDqBM;
-  p->ntiles = (N + kDqBN - 1) / kDqBN;
-  p->rm = p->rn = 0;
-  const double xb = (double)kDqBM * K * 2, wb = (double)kDqBN * K * (bits / 8.0 + 4.0 / gs);
-  double best = 0;
-  for (int gm = 1; gm <= 8; gm *= 2) {  // regions along M
-    const int gn = 8 / gm;
-    if (p->mtiles % gm || p->ntiles % gn) continue;
-    const int rm = p->mtiles / gm, rn = p->ntiles / gn;
-    const double bytes = rm * xb + rn * wb;
-    if (p->rm == 0 || bytes < best) {
-      best = bytes;
-      p->rm = rm;
-      p->rn = rn;
-    }
-  }
-  return true;
-}
-
 template <int BITS, int GS, bool F16, int MT, bool kStaged>
 int32_t launch_dq_t(hipStream_t st, const QmmArgs& a, const DqPlan& p, uint32_t lds) {
   static std::atomic<uint64_t> lds_set{0};  // this instantiation's LDS above 64 KB, per device
@@ -1079,10 +950,6 @@ __global__ __launch_bounds__(512) void qgemv1_kernel(QmmArgs a, int np, int L, i
   }
 }
 
-// Whether the one-row kernel takes this call: K / gs a power of two up to 64, or a
-// multiple of 64, and x (2 K bytes) within 64 KB of LDS.
-bool gemv1_fits(int G, int K) { return (G % 64 == 0 || (G <= 64 && (G & (G - 1)) == 0)) && K <= 32768; }
-
 template <int BITS, int GS, bool F16>
 int32_t launch_gemv1(hipStream_t st, const QmmArgs& a, int cus) {
   const int L = a.G < 64 ? a.G : 64, slots = 64 / L, gpl = a.G / L;
@@ -1099,40 +966,25 @@ int32_t launch_gemv1(hipStream_t st, const QmmArgs& a, int cus) {
 
 template <int BITS, int GS, bool F16>
 int32_t launch_t(hipStream_t st, QmmArgs a) {
+  const QmmRoute r = qmm_route(a, GS, BITS, device_cus());
+  switch (r.kernel) {
+    case QmmKernel::gemv1: return launch_gemv1<BITS, GS, F16>(st, a, device_cus());
+    case QmmKernel::qmv_ks: return launch_qmv_ks(st, a, KsPlan{r.mt, r.nt}, GS, BITS, F16);
+    case QmmKernel::qgemm_ks: return launch_qgemm_ks(st, a, KsPlan{r.mt, r.nt}, GS, BITS, F16);
+    case QmmKernel::qmv: return launch_qmv_rows<BITS, GS, F16>(st, a, r.mt, r.qmv);
+    case QmmKernel::qmvx:
+      if (r.mt == 16)
+        return r.nt == 2 ? launch_qmvx<BITS, GS, F16, 16, 2>(st, a, r.qmv) : launch_qmvx<BITS, GS, F16, 16, 1>(st, a, r.qmv);
+      return r.nt == 2 ? launch_qmvx<BITS, GS, F16, 32, 2>(st, a, r.qmv) : launch_qmvx<BITS, GS, F16, 32, 1>(st, a, r.qmv);
+    case QmmKernel::qgemm_dq:
+      return r.mt == 4   ? launch_dq<BITS, GS, F16, 4>(st, a, r.dq)
+             : r.mt == 3 ? launch_dq<BITS, GS, F16, 3>(st, a, r.dq)
+                         : launch_dq<BITS, GS, F16, 2>(st, a, r.dq);
+    case QmmKernel::qmm: break;
+  }
   int nw = a.G / 8;  // waves per workgroup: about 8 groups each, at most 8 waves
   nw = nw < 1 ? 1 : nw > kMaxWaves ? kMaxWaves : nw;
-  const int cus = device_cus();
-  if (a.M == 1 && gemv1_fits(a.G, a.K)) return launch_gemv1<BITS, GS, F16>(st, a, cus);
-  if (a.M <= 32) {
-    const KsPlan kp = plan_qmv_ks(a, BITS, cus);
-    if (kp.mt > 0) return launch_qmv_ks(st, a, kp, GS, BITS, F16);
-    const int mx = qmv_rows(a.M);
-    const QmvPlan p = plan_qmv(a.N, a.K, GS, BITS, mx, cus);
-    if (mx >= 16) {
-      // x through an LDS ring shared by the column tiles (qmv_kernel) when it reaches the
-      // wanted tile count, else x through registers (qmvx_kernel), whose LDS holds only
-      // the weights (measured: 4-bit q|k|v at 32 rows 14.9 us against 19.9; 8-bit, where
-      // only qmvx_kernel fits two tiles, 21.9 against 23.7)
-      const int want = (a.N + 15) / 16 > cus ? 2 : 1;
-      const QmvPlan px = p.NC > 0 && p.NT == want ? QmvPlan{} : plan_qmvx(a.N, a.K, GS, BITS, cus);
-      if (px.NC > 0 && (p.NC == 0 || px.NT == want)) {
-        if (mx == 16)
-          return px.NT == 2 ? launch_qmvx<BITS, GS, F16, 16, 2>(st, a, px) : launch_qmvx<BITS, GS, F16, 16, 1>(st, a, px);
-        return px.NT == 2 ? launch_qmvx<BITS, GS, F16, 32, 2>(st, a, px) : launch_qmvx<BITS, GS, F16, 32, 1>(st, a, px);
-      }
-    }
-    if (p.NC > 0) return launch_qmv_rows<BITS, GS, F16>(st, a, mx, p);
-  } else {
-    const KsPlan kp = plan_ks(a, BITS, cus);
-    if (kp.mt > 0) return launch_qgemm_ks(st, a, kp, GS, BITS, F16);
-    DqPlan dp;
-    const int mt = dq_row_tiles(a.M, a.N, a.K, cus);
-    if (plan_dq(a.M, a.N, a.K, GS, BITS, a.ldx, mt, &dp))
-      return mt == 4   ? launch_dq<BITS, GS, F16, 4>(st, a, dp)
-             : mt == 3 ? launch_dq<BITS, GS, F16, 3>(st, a, dp)
-                       : launch_dq<BITS, GS, F16, 2>(st, a, dp);
-  }
-  const int mr = a.M <= 16 ? 1 : 2;
+  const int mr = r.mt;
   a.mtiles = (a.M + 16 * mr - 1) / (16 * mr);
   const int64_t tiles = (int64_t)a.mtiles * ((a.N + 15) / 16);
   a.remap = a.mtiles > 1 && tiles % 8 == 0;

@@ -2,52 +2,18 @@
 #pragma once
 
 #include "ema_common.hpp"
+#include "qmatmul_plan.hpp"
 
 namespace ema {
 
-struct QmmArgs {
-  const uint8_t* x;  // [M, ldx] activations
-  const uint8_t* w;  // [N, K * BITS / 8] packed fields
-  const uint8_t* s;  // [N, G] scales
-  const uint8_t* b;  // [N, G] biases
-  uint8_t* y;        // [M, ldy]
-  int64_t ldx, ldy;  // row strides in elements
-  int M, N, K, G;    // G = K / GS
-  int mtiles;        // row tiles of x (16 * MR rows each)
-  int remap;         // grid size divisible by 8: give each XCD a contiguous range of tiles
-};
-
-// Time of the dequantising GEMM with 64 mt x 128 tiles, in units of 25 ns, one workgroup per
-// CU at a time: measured 6 us per round and 0.63, 0.70 and 0.84 us per 64 k at mt = 2, 3, 4.
-inline int64_t dq_cost(int M, int N, int K, int mt, int cus) {
-  const int64_t tiles = ((int64_t)M + 64 * mt - 1) / (64 * mt) * (((int64_t)N + 127) / 128);
-  return (tiles + cus - 1) / cus * (240 + (int64_t)(K / 64) * (mt == 2 ? 25 : mt == 3 ? 28 : 34));
-}
-// The mt of the least time: fewer rows per tile where that fills a last round better (M = 1531,
-// N = 6144, K = 4096: two rounds of 192 rows 106 us, of 256 rows 127; M = 520, one round: 47, 51
-// and 61 us with 128, 192 and 256 rows).
-inline int dq_row_tiles(int M, int N, int K, int cus) {
-  int best = 4;
-  for (int mt = 3; mt >= 2; --mt)
-    if (dq_cost(M, N, K, mt, cus) < dq_cost(M, N, K, best, cus)) best = mt;
-  return best;
-}
-
-// Column and row tiles of 16 of the K-split GEMM (qgemm_ks.hip); mt = 0: it does not apply.
-struct KsPlan {
-  int mt, nt;
-};
-KsPlan plan_ks(const QmmArgs& a, int bits, int cus);
+// Launches of the K-split kernels (qgemm_ks.hip): the GEMM, and exact products of up to 32 rows.
 int32_t launch_qgemm_ks(hipStream_t st, const QmmArgs& a, const KsPlan& p, int gs, int bits, bool f16);
-// The same for the exact products of up to 32 rows.
-KsPlan plan_qmv_ks(const QmmArgs& a, int bits, int cus);
 int32_t launch_qmv_ks(hipStream_t st, const QmmArgs& a, const KsPlan& p, int gs, int bits, bool f16);
 
 namespace {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kMaxWaves = 8;
 constexpr uint32_t kOffRow = 0xF0000000u;  // a buffer offset past every range: loads return 0
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_t bytes) {
@@ -93,10 +59,6 @@ constexpr uint32_t kSelLo = 0x05040100u, kSelHi = 0x07060302u;
 __device__ __forceinline__ uint32_t pair(uint32_t lo, uint32_t hi, uint32_t sel) {
   return __builtin_amdgcn_perm(hi, lo, sel);
 }
-
-// Stride, in pairs, of the rows of {scale, bias} pairs in LDS: an odd number of 16-byte
-// pieces, so that 16 rows are read without bank conflicts.
-__device__ __host__ __forceinline__ uint32_t group_stride(uint32_t G) { return ((G >> 2) | 1) << 2; }
 
 // byte I of x as f32 (v_cvt_f32_ubyteI)
 template <int I>

@@ -459,6 +459,19 @@ def test_prefill_few_rows(ema, ora, B, Hq, Hkv, T, q_off, causal, chunk):
     assert_close(got, ref, "prefill few rows")
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,T,causal,chunk", [
+    # few rows of many heads: more than 256 items of 32 rows, so 128 rows per workgroup
+    (9, 30, 3, 1, True, False), (9, 32, 4, 5, True, False), (9, 32, 4, 32, True, True), (5, 32, 4, 64, True, False),
+    (5, 20, 4, 128, False, False), (5, 16, 8, 130, False, False), (5, 16, 8, 200, True, False),
+    (4, 24, 3, 77, True, True),
+])
+def test_prefill_few_rows_of_many_heads(ema, ora, B, Hq, Hkv, T, causal, chunk):
+    say(f"prefill few rows of many heads B={B} Hq={Hq} Hkv={Hkv} T={T} causal={causal} chunk={chunk}")
+    got, ref = _prefill_case(ema, ora, B, Hq, Hkv, 128, 512, T, [0, 37, 300, 129, 1, 64, 63, 200, 5][:B], causal, chunk,
+                             seed=345 + T + B)
+    assert_close(got, ref, "prefill few rows of many heads")
+
+
 @pytest.mark.parametrize("causal,chunk", [(True, False), (False, False), (True, True)])
 def test_prefill_xcd_grid_mapping(ema, ora, causal, chunk):
     """batch x kv heads a multiple of 8 (the XCD-grouped grid order), ragged offsets."""
@@ -531,21 +544,26 @@ def test_prefill_chunk_on_existing_cache_every_block(ema, ora):
 
 @pytest.mark.parametrize("causal,chunk,q_off", [(True, True, 100), (True, True, 64), (False, True, 37),
                                                 (True, False, 150), (False, False, 0)])
-def test_prefill_ignores_cache_rows_outside_the_window(ema, ora, causal, chunk, q_off):
+@pytest.mark.parametrize("B,Hq,Hkv,T", [
+    (1, 4, 2, 120),   # 32 query rows per workgroup
+    (5, 16, 8, 120),  # 128, one query block per workgroup
+    (6, 32, 8, 300),  # two (paired)
+])
+def test_prefill_ignores_cache_rows_outside_the_window(ema, ora, B, Hq, Hkv, T, causal, chunk, q_off):
     """NaN in every cache row outside [kv_begin, kv_len) (before a chunk-only window and
     past the valid length) gives bit-identical output to finite data there: the
     reference attends over a slice of the cache (crates/serve/src/forward_qwen3.rs:150),
     so those rows are never read."""
     import torch
 
-    B, Hq, Hkv, D, cap, T = 1, 4, 2, 128, 512, 120
-    say(f"prefill NaN outside window causal={causal} chunk={chunk} q_off={q_off}")
+    D, cap = 128, 512
+    say(f"prefill NaN outside window B={B} Hq={Hq} T={T} causal={causal} chunk={chunk} q_off={q_off}")
     q = ora.normal_bf16((B, Hq, T, D), seed=360)
     kc = ora.normal_bf16((B, Hkv, cap, D), seed=361)
     vc = ora.normal_bf16((B, Hkv, cap, D), seed=362)
     kv_len = q_off + T
     lo = q_off if chunk else 0
-    qo = np.asarray([q_off], np.int32)
+    qo = np.full(B, q_off, np.int32)
 
     def run(k, v):
         out = host(ema.prefill_attention(dev(q), make_cache(ema, k, v), dev(qo), causal=causal, chunk_only=chunk))
@@ -559,7 +577,7 @@ def test_prefill_ignores_cache_rows_outside_the_window(ema, ora, causal, chunk, 
         a[:, :, :lo] = 0x7FC0
     dirty = run(kp, vp)
     assert np.array_equal(clean, dirty)
-    ref = ora.sdpa(q, kc, vc, np.asarray([kv_len]), scale_of(D), causal, kv_begin=np.asarray([lo]) if chunk else None)
+    ref = ora.sdpa(q, kc, vc, np.full(B, kv_len), scale_of(D), causal, kv_begin=np.full(B, lo) if chunk else None)
     assert_close(clean, ref, "prefill window")
 
 

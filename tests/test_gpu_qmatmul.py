@@ -97,8 +97,7 @@ def test_qmatmul_matches_oracle(ema, ora, dtype, bits, gs):
                                       (16, 6144, 8), (32, 6144, 8), (32, 4096, 8)])
 def test_qmatmul_qwen3_8b_qkv_decode_shape(ema, ora, M, N, bits):
     # x [M, 4096] -> q|k|v [M, 6144] or o_proj [M, 4096], group 64: the one-row kernel (M = 1)
-    # and the staged kernel with one or two column tiles (chosen by the tile count; 8-bit
-    # weights of 32 rows take most of the LDS)
+    # and the K-split kernel with one or two column tiles
     K, gs = 4096, 64
     say(f"qmatmul Qwen3-8B decode shape M={M} N={N} K={K} bits={bits}")
     d, h = make(ora, 1, M, N, K, gs, bits)
@@ -130,9 +129,9 @@ def test_qmatmul_one_row_8bit_group_128_many_rows(ema, ora, dtype):
 
 
 @pytest.mark.parametrize("M,gs,dtype", [(20, 128, "bf16"), (12, 64, "f16")])
-def test_qmatmul_8bit_wide_rows_x_in_registers(ema, ora, M, gs, dtype):
-    # 8-bit weights of two 16-row column tiles fill most of the LDS, so x streams through
-    # registers (qmvx_kernel); ragged rows of x
+def test_qmatmul_8bit_wide_rows(ema, ora, M, gs, dtype):
+    # 8-bit weights, more column tiles than CUs: the K-split kernel, two column tiles; ragged
+    # rows of x (test_qmatmul_scales_off_alignment runs the staged kernels at these sizes)
     N, K, bits = 6144, 4096, 8
     say(f"qmatmul 8-bit M={M} N={N} K={K} gs={gs} {dtype}")
     d, h = make(ora, 60 + M, M, N, K, gs, bits, dtype)
@@ -160,100 +159,162 @@ def test_qmatmul_prefill_rows(ema, ora, M, N, K, gs, bits, dtype):
     check(ora, y, h, gs, bits, f"M={M}", dtype)
 
 
-@pytest.mark.parametrize("M,N,K,gs,bits,dtype", [
-    # the K-split GEMM: each of its tiles (row x column tiles of 16, chosen by the number of
-    # tiles on 256 CUs), ragged last rows and columns, fewer units of 128 k than waves
-    (33, 100, 128, 32, 4, "bf16"),      # 3 x 2, one unit
-    (48, 30, 384, 32, 8, "f16"),        # 3 x 2, three units
-    (64, 5100, 256, 64, 4, "f16"),      # 4 x 2
-    (157, 4093, 256, 64, 4, "bf16"),    # 5 x 2
-    (157, 4090, 512, 128, 8, "bf16"),   # 5 x 2
-    (96, 6140, 256, 64, 8, "bf16"),     # 3 x 3
-    (101, 6144, 256, 32, 4, "bf16"),    # 4 x 3
-    (127, 6143, 256, 32, 8, "f16"),     # 4 x 3
-    (159, 6142, 512, 128, 4, "f16"),    # 5 x 3
-    (140, 5437, 256, 64, 4, "bf16"),    # 3 x 4
-    (140, 5440, 256, 64, 8, "f16"),     # 3 x 4
-    (190, 5439, 256, 32, 4, "bf16"),    # 4 x 4
-    (80, 64, 1152, 64, 4, "bf16"),      # nine units: one wave takes two
-    (50, 70, 2560, 64, 8, "bf16"),      # twenty units
-])
-def test_qmatmul_ksplit_tiles(ema, ora, M, N, K, gs, bits, dtype):
-    import torch
+# The last column is the kernel and its tiles on 256 CUs, which tests/test_qmm_route.py checks on
+# the CPU against the rules that the launches use.
+KSPLIT_TILES = [
+    # the K-split GEMM: each of its tiles (row x column tiles of 16), ragged last rows and
+    # columns, at most one unit of 128 k per wave
+    (33, 100, 128, 32, 4, "bf16", "qgemm_ks 3 2"),      # one unit
+    (48, 30, 384, 32, 8, "f16", "qgemm_ks 3 2"),        # three units
+    (64, 5100, 256, 64, 4, "f16", "qgemm_ks 4 2"),
+    (157, 4093, 256, 64, 4, "bf16", "qgemm_ks 5 2"),
+    (157, 4090, 512, 128, 8, "bf16", "qgemm_ks 5 2"),
+    (96, 6140, 256, 64, 8, "bf16", "qgemm_ks 3 3"),
+    (101, 6144, 256, 32, 4, "bf16", "qgemm_ks 4 3"),
+    (127, 6143, 256, 32, 8, "f16", "qgemm_ks 4 3"),
+    (159, 6142, 512, 128, 4, "f16", "qgemm_ks 5 3"),
+    (140, 5437, 256, 64, 4, "bf16", "qgemm_ks 3 4"),
+    (140, 5440, 256, 64, 8, "f16", "qgemm_ks 3 4"),
+    (190, 5439, 256, 32, 4, "bf16", "qgemm_ks 4 4"),
+    # each tile again with several units per wave (the refill of the next unit, the walk's wrap
+    # at the end of K, slots written again), equal and unequal shares of the waves
+    (80, 64, 1152, 32, 4, "bf16", "qgemm_ks 3 2"),      # nine units: one wave takes two
+    (50, 70, 2560, 64, 8, "bf16", "qgemm_ks 3 2"),      # twenty units
+    (64, 5100, 1152, 32, 4, "bf16", "qgemm_ks 4 2"),
+    (61, 5437, 2176, 32, 8, "bf16", "qgemm_ks 4 2"),
+    (157, 4096, 4096, 64, 4, "bf16", "qgemm_ks 5 2"),
+    (157, 4093, 2304, 64, 8, "f16", "qgemm_ks 5 2"),
+    (96, 5437, 2304, 64, 4, "f16", "qgemm_ks 3 3"),
+    (93, 6140, 1152, 32, 8, "bf16", "qgemm_ks 3 3"),
+    (127, 6140, 2176, 32, 4, "bf16", "qgemm_ks 4 3"),
+    (125, 6144, 2304, 64, 8, "bf16", "qgemm_ks 4 3"),
+    (157, 6144, 4096, 64, 4, "bf16", "qgemm_ks 5 3"),
+    (140, 5437, 2304, 64, 4, "f16", "qgemm_ks 3 4"),
+    (139, 5440, 1152, 32, 8, "bf16", "qgemm_ks 3 4"),
+    (190, 5437, 2176, 32, 4, "bf16", "qgemm_ks 4 4"),
+    (40, 64, 9728, 32, 4, "bf16", "qgemm_ks 3 2"),      # 304 groups: scales staged in two passes
+    (40, 70, 9728, 32, 8, "f16", "qgemm_ks 3 2"),
+]
 
-    say(f"qmatmul K-split M={M} N={N} K={K} gs={gs} bits={bits} {dtype}")
-    d, h = make(ora, M + N + K, M, N, K, gs, bits, dtype)
-    y = ema.quantized_matmul(*d, group_size=gs, bits=bits)
-    check(ora, y, h, gs, bits, f"M={M}", dtype)
-    # into a view with an odd row stride (2-byte stores): the same bits, nothing beside them
-    wide = torch.full((M, N + 3), 7.0, dtype=y.dtype, device="cuda")
-    ema.quantized_matmul(*d, group_size=gs, bits=bits, out=wide[:, 1:N + 1])
-    torch.cuda.synchronize()
-    assert torch.equal(wide[:, 1:N + 1].contiguous().view(torch.int16), y.view(torch.int16))
-    assert torch.all(wide[:, :1] == 7.0) and torch.all(wide[:, N + 1:] == 7.0)
+KSPLIT_DECODE = [
+    # exact products split over K (K >= 2048; 8 bits and up to 16 rows K >= 4096): 8, 16 and 32
+    # rows, one and two column tiles, ragged columns, units that do not divide among the eight
+    # waves
+    (2, 70, 2048, 64, 4, "bf16", "qmv_ks 1 1"),
+    (8, 33, 2176, 32, 4, "f16", "qmv_ks 1 1"),          # 17 units
+    (9, 100, 4096, 128, 8, "bf16", "qmv_ks 1 1"),
+    (16, 4099, 2048, 64, 4, "bf16", "qmv_ks 1 2"),      # ragged
+    (17, 48, 2560, 64, 8, "f16", "qmv_ks 2 1"),         # 20 units
+    (31, 4110, 2304, 32, 4, "bf16", "qmv_ks 2 2"),      # 18 units
+    (32, 8200, 2048, 64, 4, "bf16", "qmv_ks 2 1"),      # more than two rounds: one column tile
+    (5, 4097, 4608, 64, 8, "bf16", "qmv_ks 1 2"),       # 36 units: a fifth turn for four waves
+    (4, 40, 9728, 32, 4, "f16", "qmv_ks 1 1"),          # 304 groups: scales staged in two passes
+    # calls that stay with the staged kernels: short K with one and two column tiles, 8 bits and
+    # up to 16 rows below K = 4096, 384 groups (past the LDS bound of the K-split kernel)
+    (16, 4112, 1024, 64, 4, "bf16", "qmv 16 2"),
+    (32, 4109, 1024, 64, 4, "f16", "qmv 32 2"),
+    (8, 4100, 1024, 32, 4, "bf16", "qmv 8 2"),
+    (9, 100, 3072, 64, 8, "bf16", "qmv 16 1"),
+    (16, 6144, 2560, 64, 8, "bf16", "qmv 16 2"),
+    (3, 40, 12288, 32, 4, "bf16", "qmv 4 1"),
+    (17, 40, 14848, 32, 4, "bf16", "qmvx 32 1"),
+    (9, 100, 3968, 128, 8, "bf16", "qmm 1 1"),          # 31 groups: the streaming kernel
+]
 
-
-@pytest.mark.parametrize("M,N,K,gs,bits,dtype", [
-    # exact products split over K (K >= 2048; 8 bits and up to 16 rows K >= 4096): 8, 16 and 32 rows, one and two column tiles,
-    # ragged columns, units that do not divide among the eight waves
-    (2, 70, 2048, 64, 4, "bf16"),
-    (8, 33, 2176, 32, 4, "f16"),        # 17 units
-    (9, 100, 4096, 128, 8, "bf16"),
-    (9, 100, 3968, 128, 8, "bf16"),     # 8 bits, up to 16 rows, below K = 4096: the staged kernel
-    (16, 4099, 2048, 64, 4, "bf16"),    # two column tiles, ragged
-    (17, 48, 2560, 64, 8, "f16"),       # 20 units
-    (31, 4110, 2304, 32, 4, "bf16"),    # two column tiles, 18 units
-    (32, 8200, 2048, 64, 4, "bf16"),    # more than two rounds: one column tile
-    (5, 4097, 4608, 64, 8, "bf16"),     # 36 units: a fifth turn for four waves
-    (3, 40, 12288, 32, 4, "bf16"),      # 384 groups: past the LDS bound, the staged kernels
-    (4, 40, 9728, 32, 4, "f16"),        # 304 groups: scales staged in two passes
-])
-def test_qmatmul_ksplit_decode_rows(ema, ora, M, N, K, gs, bits, dtype):
-    import torch
-
-    say(f"qmatmul K-split decode M={M} N={N} K={K} gs={gs} bits={bits} {dtype}")
-    d, h = make(ora, M + N + K, M, N, K, gs, bits, dtype)
-    y = ema.quantized_matmul(*d, group_size=gs, bits=bits)
-    check(ora, y, h, gs, bits, f"M={M}", dtype)
-    wide = torch.full((M, N + 3), 7.0, dtype=y.dtype, device="cuda")
-    ema.quantized_matmul(*d, group_size=gs, bits=bits, out=wide[:, 1:N + 1])
-    torch.cuda.synchronize()
-    assert torch.equal(wide[:, 1:N + 1].contiguous().view(torch.int16), y.view(torch.int16))
-    assert torch.all(wide[:, :1] == 7.0) and torch.all(wide[:, N + 1:] == 7.0)
-
-
-@pytest.mark.parametrize("M,N,K,gs,bits,dtype", [
+DQ_TILES = [
     # tiles of 128, 192 and 256 rows of the dequantising GEMM (chosen by the rounds on 256 CUs),
     # ragged in both directions, scales staged in LDS or loaded per chunk (K / gs odd)
-    (1020, 4093, 128, 32, 4, "bf16"),   # 256 tiles of 128 rows
-    (1000, 4096, 192, 64, 8, "f16"),    # the same, three groups: loaded per chunk
-    (1530, 4090, 256, 32, 8, "bf16"),   # 256 tiles of 192 rows
-    (1531, 4096, 192, 64, 4, "f16"),
-    (2040, 4091, 128, 32, 4, "f16"),    # 256 tiles of 256 rows
-    (2047, 4096, 64, 64, 8, "bf16"),    # one chunk
-])
-def test_qmatmul_dequantising_tiles(ema, ora, M, N, K, gs, bits, dtype):
+    (1020, 4093, 128, 32, 4, "bf16", "qgemm_dq 2 1"),   # 256 tiles of 128 rows
+    (1000, 4096, 192, 64, 8, "f16", "qgemm_dq 2 1"),    # the same, three groups: loaded per chunk
+    (1530, 4090, 256, 32, 8, "bf16", "qgemm_dq 3 1"),   # 256 tiles of 192 rows
+    (1531, 4096, 192, 64, 4, "f16", "qgemm_dq 3 1"),
+    (2040, 4091, 128, 32, 4, "f16", "qgemm_dq 4 1"),    # 256 tiles of 256 rows
+    (2047, 4096, 64, 64, 8, "bf16", "qgemm_dq 4 1"),    # one chunk
+]
+
+# Scales and biases that start 4 or 2 bytes past a 16-byte boundary (the entry asks for their
+# element's alignment only): the K-split kernels and the staged scales of the dequantising GEMM
+# need 8 bytes.
+OFF_ALIGNMENT = [
+    (20, 6144, 4096, 128, 8, "bf16", 4, "qmvx 32 2"),
+    (12, 6144, 4096, 64, 8, "f16", 4, "qmv 16 2"),
+    (32, 4096, 4096, 64, 8, "bf16", 4, "qmv 32 1"),
+    (157, 4093, 1024, 64, 4, "bf16", 4, "qgemm_dq 2 1"),
+    (157, 300, 1024, 64, 8, "f16", 2, "qgemm_dq 2 1"),
+]
+
+
+def same_bits_elsewhere(ema, d, y, gs, bits):
+    """The call again into a view with an odd row stride (2-byte stores) and from rows of x that
+    lie further apart: the same bits, nothing written beside the view."""
     import torch
 
-    say(f"qmatmul dequantising tiles M={M} N={N} K={K} gs={gs} bits={bits} {dtype}")
-    d, h = make(ora, M + N + K, M, N, K, gs, bits, dtype)
-    y = ema.quantized_matmul(*d, group_size=gs, bits=bits)
-    check(ora, y, h, gs, bits, f"M={M}", dtype)
+    M, N, K = y.shape[0], y.shape[1], d[0].shape[1]
     wide = torch.full((M, N + 3), 7.0, dtype=y.dtype, device="cuda")
     ema.quantized_matmul(*d, group_size=gs, bits=bits, out=wide[:, 1:N + 1])
+    wx = torch.full((M, K + 72), float("nan"), dtype=y.dtype, device="cuda")
+    wx[:, :K] = d[0]
+    strided = ema.quantized_matmul(wx[:, :K], *d[1:], group_size=gs, bits=bits)
     torch.cuda.synchronize()
     assert torch.equal(wide[:, 1:N + 1].contiguous().view(torch.int16), y.view(torch.int16))
     assert torch.all(wide[:, :1] == 7.0) and torch.all(wide[:, N + 1:] == 7.0)
+    assert torch.equal(strided.view(torch.int16), y.view(torch.int16))
 
 
-@pytest.mark.parametrize("M", [1, 32, 256])
-def test_qmatmul_graph_replay(ema, ora, M):
+@pytest.mark.parametrize("M,N,K,gs,bits,dtype,route", KSPLIT_TILES)
+def test_qmatmul_ksplit_tiles(ema, ora, M, N, K, gs, bits, dtype, route):
+    say(f"qmatmul K-split M={M} N={N} K={K} gs={gs} bits={bits} {dtype} ({route})")
+    d, h = make(ora, M + N + K, M, N, K, gs, bits, dtype)
+    y = ema.quantized_matmul(*d, group_size=gs, bits=bits)
+    check(ora, y, h, gs, bits, f"M={M}", dtype)
+    same_bits_elsewhere(ema, d, y, gs, bits)
+
+
+@pytest.mark.parametrize("M,N,K,gs,bits,dtype,route", KSPLIT_DECODE)
+def test_qmatmul_ksplit_decode_rows(ema, ora, M, N, K, gs, bits, dtype, route):
+    say(f"qmatmul K-split decode M={M} N={N} K={K} gs={gs} bits={bits} {dtype} ({route})")
+    d, h = make(ora, M + N + K, M, N, K, gs, bits, dtype)
+    y = ema.quantized_matmul(*d, group_size=gs, bits=bits)
+    check(ora, y, h, gs, bits, f"M={M}", dtype)
+    same_bits_elsewhere(ema, d, y, gs, bits)
+
+
+@pytest.mark.parametrize("M,N,K,gs,bits,dtype,route", DQ_TILES)
+def test_qmatmul_dequantising_tiles(ema, ora, M, N, K, gs, bits, dtype, route):
+    say(f"qmatmul dequantising tiles M={M} N={N} K={K} gs={gs} bits={bits} {dtype} ({route})")
+    d, h = make(ora, M + N + K, M, N, K, gs, bits, dtype)
+    y = ema.quantized_matmul(*d, group_size=gs, bits=bits)
+    check(ora, y, h, gs, bits, f"M={M}", dtype)
+    same_bits_elsewhere(ema, d, y, gs, bits)
+
+
+@pytest.mark.parametrize("M,N,K,gs,bits,dtype,past,route", OFF_ALIGNMENT)
+def test_qmatmul_scales_off_alignment(ema, ora, M, N, K, gs, bits, dtype, past, route):
+    import torch
+
+    say(f"qmatmul scales {past} bytes past 16 M={M} N={N} K={K} gs={gs} bits={bits} {dtype} ({route})")
+    d, h = make(ora, M + N + K + past, M, N, K, gs, bits, dtype)
+
+    def shifted(t):
+        flat = torch.empty(t.numel() + past // 2, dtype=t.dtype, device="cuda")
+        v = flat[past // 2:].view(t.shape)
+        v.copy_(t)
+        assert v.data_ptr() % 16 == past
+        return v
+
+    y = ema.quantized_matmul(d[0], d[1], shifted(d[2]), shifted(d[3]), group_size=gs, bits=bits)
+    check(ora, y, h, gs, bits, f"M={M}", dtype)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 192, 1024), (32, 192, 1024), (256, 192, 1024), (1000, 4096, 192),
+                                   (16, 4099, 4096), (32, 4096, 4096), (157, 4096, 2304)])
+def test_qmatmul_graph_replay(ema, ora, M, N, K):
     # captured in a HIP graph and replayed several times with eager work between the
     # replays: every replay equals the eager call (no memsets or host state in the call)
     import torch
 
-    N, K, gs, bits = 192, 1024, 64, 4
-    say(f"qmatmul graph replay M={M}")
+    gs, bits = 64, 4
+    say(f"qmatmul graph replay M={M} N={N} K={K}")
     d, _ = make(ora, 5 + M, M, N, K, gs, bits)
     y_eager = ema.quantized_matmul(*d, group_size=gs, bits=bits)
     torch.cuda.synchronize()

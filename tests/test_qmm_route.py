@@ -1,0 +1,51 @@
+"""CPU check of the rules that choose a quantised projection's kernel and tiles
+(engine-mlx_amd/csrc/qmatmul_plan.hpp, the definitions that the launches use): every case of the
+GPU tests whose kernel its comment names runs that kernel on 256 CUs, every kernel and tile has
+such a case, and a call's arithmetic (exact products, or weights dequantised into the activation
+type) depends on its rows and K alone."""
+import os
+import subprocess
+
+import pytest
+
+import test_gpu_qmatmul as cases
+
+CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
+
+
+@pytest.fixture(scope="module")
+def routes():
+    subprocess.run(["make", "-s", "-C", CPP, "test_qmm_route"], check=True)
+
+    def run(calls):
+        """calls: (M, N, K, group, bits, ldx, bytes of scales past 16, CUs)"""
+        text = "\n".join(" ".join(str(v) for v in c) for c in calls) + "\n"
+        r = subprocess.run([os.path.join(CPP, "test_qmm_route")], input=text, capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stderr
+        out = r.stdout.strip().split("\n")
+        assert len(out) == len(calls)
+        return out
+
+    return run
+
+
+def test_gpu_cases_run_the_kernel_they_name(routes):
+    listed = [(c[:5], 0, c[6]) for c in cases.KSPLIT_TILES + cases.KSPLIT_DECODE + cases.DQ_TILES]
+    listed += [(c[:5], c[6], c[7]) for c in cases.OFF_ALIGNMENT]
+    got = routes([(*c, c[2], past, 256) for c, past, _ in listed])
+    for (c, past, want), r in zip(listed, got):
+        assert r == want, f"{c}, scales {past} bytes past 16: {r}, not {want}"
+
+
+def units(K):
+    return K // 128
+
+
+def test_every_tile_has_a_case_of_its_main_loop(routes):
+    """Each tile of the K-split GEMM that the rules can choose is tested with several units per
+    wave, at 4 and at 8 bits."""
+    calls = [(M, N, K, 32, bits, K, 0, 256) for M in range(33, 700, 9) for N in range(64, 9000, 331)
+             for K in (1152, 4096) for bits in (4, 8)]
+    chosen = {(c[4], r) for c, r in zip(calls, routes(calls)) if r.startswith("qgemm_ks")}
+    tested = {(c[4], c[6]) for c in cases.KSPLIT_TILES if units(c[2]) > 8}
+    assert chosen == tested, chosen ^ tested

@@ -50,12 +50,17 @@ struct DqPlan {
   int rm, rn;  // tile rows / columns per region (regions: mtiles / rm x ntiles / rn = 8), or 0
 };
 
+// Whether 256 rows of x lie within one buffer range: the row stride up to which a call of more
+// than 32 rows takes dequantised weights. One line for every tile height and for the K-split GEMM,
+// so that the arithmetic of a call does not depend on which of them its sizes choose.
+inline bool dq_x_fits(int64_t ldx, int K) { return 256 * ldx * 2 + (int64_t)K * 2 < ((int64_t)1 << 31); }
+
 // Plan of the dequantising GEMM: K a multiple of the chunk and of the group, x within one
 // buffer range per tile. Regions: 2 x 4, 4 x 2, 1 x 8 or 8 x 1 whole tile rows and columns,
 // the one with the least bytes per region, when the grid divides into them.
 inline bool plan_dq(int M, int N, int K, int gs, int bits, int64_t ldx, int mt, DqPlan* p) {
   const int kDqBM = 64 * mt;
-  if (K % kDqKC || K % gs || (int64_t)kDqBM * ldx * 2 + (int64_t)K * 2 >= ((int64_t)1 << 31)) return false;
+  if (K % kDqKC || K % gs || !dq_x_fits(ldx, K)) return false;
   p->mtiles = (M + kDqBM - 1) / kDqBM;
   p->ntiles = (N + kDqBN - 1) / kDqBN;
   p->rm = p->rn = 0;
@@ -92,7 +97,7 @@ constexpr bool ks_tile(int bits, int mt, int nt) {
 }
 
 // Whole units, four groups' scales or biases per 8-byte load, the pairs of 64 rows and the
-// slots within the LDS, 32-bit offsets inside a tile of 80 rows.
+// slots within the LDS, 32-bit offsets inside a tile of 80 rows (the GEMM: dq_x_fits also).
 inline bool ks_fits(const QmmArgs& a) {
   return a.K % kUnit == 0 && a.G % 4 == 0 && (((uintptr_t)a.s | (uintptr_t)a.b) & 7) == 0 &&
          (a.G + 4) * 64 * 4 + kKsSlotBytes <= kKsMaxLds &&
@@ -109,7 +114,7 @@ inline bool ks_fits(const QmmArgs& a) {
 // 39.9 against 23.8 at 2048 (8 MB).
 inline KsPlan plan_ks(const QmmArgs& a, int bits, int cus) {
   KsPlan best{0, 0};
-  if (!ks_fits(a) || (int64_t)a.M * a.K * 2 > (5 << 20)) return best;
+  if (!ks_fits(a) || !dq_x_fits(a.ldx, a.K) || (int64_t)a.M * a.K * 2 > (5 << 20)) return best;
   auto rounds = [&](int rows, int cols) {
     return (((int64_t)a.M + rows - 1) / rows * (((int64_t)a.N + cols - 1) / cols) + cus - 1) / cus;
   };

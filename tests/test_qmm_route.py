@@ -49,3 +49,14 @@ def test_every_tile_has_a_case_of_its_main_loop(routes):
     chosen = {(c[4], r) for c, r in zip(calls, routes(calls)) if r.startswith("qgemm_ks")}
     tested = {(c[4], c[6]) for c in cases.KSPLIT_TILES if units(c[2]) > 8}
     assert chosen == tested, chosen ^ tested
+
+
+def test_arithmetic_depends_on_rows_and_k_alone(routes):
+    """More than 32 rows and K a multiple of 64: dequantised weights whatever the tile, up to the
+    row stride at which 256 rows pass the 2 GiB of a buffer range; beyond it exact products."""
+    strides = (0, 72, 4_000_000, 4_186_000, 4_194_304, 5_000_000, 8_000_000, 13_000_000, 30_000_000)
+    calls = [(M, N, K, gs, bits, max(K, s), past, 256) for M in (33, 157, 300, 1531) for N in (100, 4096, 6144)
+             for K in (256, 320, 4096) for gs, bits in ((32, 8), (64, 4)) for s in strides for past in (0, 2)]
+    for c, r in zip(calls, routes(calls)):
+        dequantised = 256 * c[5] * 2 + c[2] * 2 < 1 << 31
+        assert (r.split()[0] in ("qgemm_ks", "qgemm_dq")) == dequantised, (c, r)

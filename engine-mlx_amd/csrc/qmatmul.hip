@@ -780,30 +780,26 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
 #pragma unroll
       for (int rt = 0; rt < MT; ++rt)
 #pragma unroll
-        for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = mma<F16>(B[ct], A[rt], acc[rt][ct]);
+        for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = mma<F16>(A[rt], B[ct], acc[rt][ct]);
     }
     __syncthreads();
   }
 
-  // (weights, x) products: lane (r16, j) of tile (rt, ct) holds columns 4 j .. 4 j + 3 of row
-  // r16
-  const bool wide = (((uintptr_t)a.y | (uint64_t)a.ldy * 2) & 7) == 0;
+  // (x, weights) products: lane (r16, j) of tile (rt, ct) holds rows 4 j .. 4 j + 3 of column
+  // r16, and a 2-byte store writes 32 bytes of four rows. With the operands the other way round,
+  // so that a lane holds four columns of a row and stores 8 bytes (32 bytes of 16 rows), a round
+  // of workgroups took 1.5 to 2 us more: M = 1000, N = 6144 16.8 us against 14.8 at K = 512, 65
+  // against 62 at K = 4096.
 #pragma unroll
   for (int rt = 0; rt < MT; ++rt)
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
-      const int m = 16 * MT * wm + 16 * rt + (int)r16, n = 64 * wn + 16 * ct + 4 * (int)j;
-      if (m >= rows_m || n >= rows_n) continue;
-      uint16_t* const y = reinterpret_cast<uint16_t*>(a.y) + (int64_t)(m0 + m) * a.ldy + n0 + n;
-      const f32x4 v = acc[rt][ct];
-      if (wide && n + 4 <= rows_n) {
-        *reinterpret_cast<u32x2*>(y) = u32x2{pack_act2<F16>(v[0], v[1]), pack_act2<F16>(v[2], v[3])};
-      } else {
+    for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (n + q < rows_n) y[q] = f32_to_act<F16>(v[q]);
+      for (int q = 0; q < 4; ++q) {
+        const int m = 16 * MT * wm + 16 * rt + 4 * (int)j + q, n = 64 * wn + 16 * ct + (int)r16;
+        if (m < rows_m && n < rows_n)
+          reinterpret_cast<uint16_t*>(a.y)[(int64_t)(m0 + m) * a.ldy + n0 + n] = f32_to_act<F16>(acc[rt][ct][q]);
       }
-    }
 }
 
 template <int BITS, int GS, bool F16, int MT, bool kStaged>

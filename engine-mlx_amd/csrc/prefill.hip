@@ -218,6 +218,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     return kSeg == 1 || (kSeg == 0 && kPair && j < n1);
   };
   const int offB = gbB - n1;
+  const int n1_edge = kPair && kv_begin % kBN ? n1 - 2 : n1;
   auto blk_of = [&](int j) __attribute__((always_inline)) { return j + (in_a(j, SegAny{}) ? gbA : offB); };
 
   const int hh = lane >> 5;                       // which half of the k slots
@@ -494,7 +495,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       // packed bf16 words read as f16 pairs: for p >= 0 the bit patterns below 0x7C00 are
       // ordered alike in both formats, and larger ones (p >= 2^121, inf, NaN) read as f16
       // inf or NaN, which the maximum keeps.
-      bool fast = all_seen;
+      // (not in segment A's last steps when a window begins inside a block: they load segment
+      // B's first block, that block again, and only load_k / load_v leave out its early rows)
+      bool fast = all_seen && !(kMask && decltype(seg)::value == 1 && j >= n1_edge);
       if (fast) {
         const uint32_t kob = blk_off(j + 2), vob = blk_off(j + 1);
         const int kwrap = wrap_rows(j + 2), vwrap = wrap_rows(j + 1);
@@ -638,7 +641,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       const uint16_t* qp = light_q(32 * wq) + k_lane;
       for (int s = 0; s < 8; ++s) qop[s] = scale_q(*(const u32x4*)(qp + (k_x ^ (16 * s))));
       const int actA = seg_act(gbA, wfaA, n1), maskA = seg_mask(gbA, wfaA);
-      const int tfA = actA < maskA ? actA : maskA;
+      const int tfA = actA < maskA ? (actA < n1_edge ? actA : n1_edge) : (maskA < n1_edge ? maskA : n1_edge);
       for (; t < n1 - 1 && t < 1; ++t) half0(t, false, mask_on, SegA{}, false);
       for (; t < n1 - 1 && t < tfA; ++t) half0(t, true, mask_off, SegA{}, false);
       for (; t < n1 - 1; ++t) half0(t, false, mask_on, SegA{}, false);

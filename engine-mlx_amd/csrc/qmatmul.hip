@@ -551,7 +551,7 @@ int32_t launch_qmv_rows(hipStream_t st, const QmmArgs& a, int mx, const QmvPlan&
 //   chunks ahead into registers (three sets in turn), then write x into LDS and dequantise
 //   the weights into it, w = round(fma(s, q, b)) in f32 then to bf16 / f16 (the rounding
 //   of MLX's dequantise, parity unpinned as to one rounding or two). Staging the scales and
-//   biases of all of K in LDS instead was slower over 900 shapes (1.5 % together, up to 14 %
+//   biases of all of K in LDS instead was slower over 900 shapes (2 % together, up to 14 %
 //   with 128-row tiles, whose two workgroups per CU the pairs' LDS makes one).
 // Two LDS buffers: the loaders fill chunk c + 1's while the compute waves multiply chunk
 // c's, one barrier per chunk. The loaders issue every load on every path (a chunk past the

@@ -251,6 +251,28 @@ inline int qmv_rows(int M) { return M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 
 // multiple of 64, and x (2 K bytes) within 64 KB of LDS.
 inline bool gemv1_fits(int G, int K) { return (G % 64 == 0 || (G <= 64 && (G & (G - 1)) == 0)) && K <= 32768; }
 
+// Up to 32 rows, K of 2048 to 3072 and more columns than one round of workgroups holds: whether
+// the kernels that keep a column tile's weights in LDS (one to three chunks at such K) are faster
+// than the K-split kernel, each of whose waves has two or three units per workgroup to set against
+// its fixed 3.5 us. r1, r2: rounds of workgroups with one and two column tiles each (K-split: one;
+// the staged kernel: one up to 4 rows, two above, so that it gains where r2 is just full).
+// Measured, us, K-split / staged, 4 bits, group 64: K = 2048, N = 151936 81.5 / 54.9 at 2 rows,
+// 85.0 / 59.1 at 8; N = 16384 18.7 / 17.0 at 24; N = 9216 at 24 1.13 times faster split. 8 bits: K =
+// 2048, N = 32768, 32 rows 51.5 / 37.2; K = 2560 60.2 / 48.2. From K = 4096 on it is faster at
+// every N.
+inline bool staged_fills_rounds(int M, int N, int K, int gs, int bits, int cus) {
+  const int t1 = (N + 15) / 16, t2 = (N + 31) / 32;
+  if (t2 <= cus) return false;
+  const int r1 = (t1 + cus - 1) / cus, r2 = (t2 + cus - 1) / cus;
+  const bool even = r1 >= 2 * r2 || r1 > 12;
+  if (M <= 2) return r1 > (K <= 2048 ? 2 : K == 2560 ? 20 : K == 3072 ? 6 : N);
+  if (M <= 4) return K <= 2048 && r1 > 3;
+  if (M <= 8) return K <= 2048 && r1 > 3;
+  if (M <= 16) return K <= 2048 && gs >= 64 && even;
+  if (bits == 4) return K <= 2048 ? (gs == 32 ? r1 > 3 : even) : K <= 3072 && gs == 32 && even;
+  return K <= 2048 || (K <= 2560 && r1 > (gs == 128 ? 2 : 3)) || (K <= 3072 && gs <= 64 && r1 > 7 && even);
+}
+
 enum class QmmKernel { gemv1, qmv_ks, qgemm_ks, qmv, qmvx, qgemm_dq, qmm };
 struct QmmRoute {
   QmmKernel kernel;
@@ -265,21 +287,14 @@ inline QmmRoute qmm_route(const QmmArgs& a, int gs, int bits, int cus) {
     return r;
   }
   if (a.M <= 32) {
-    const KsPlan kp = plan_qmv_ks(a, bits, cus);
-    if (kp.mt > 0) {
-      r.kernel = QmmKernel::qmv_ks;
-      r.mt = kp.mt;
-      r.nt = kp.nt;
-      return r;
-    }
     const int mx = qmv_rows(a.M);
     QmvPlan p = plan_qmv(a.N, a.K, gs, bits, mx, cus);
     QmmKernel kernel = QmmKernel::qmv;
     if (mx >= 16) {
       // x through an LDS ring shared by the column tiles (qmv_kernel) when it reaches the
       // wanted tile count, else x through registers (qmvx_kernel), whose LDS holds only
-      // the weights (measured: 4-bit q|k|v at 32 rows 14.9 us against 19.9; 8-bit, where
-      // only qmvx_kernel fits two tiles, 21.9 against 23.7)
+      // the weights (8 bits, N = 6144, K = 4096, 32 rows, scales that are not 8-byte aligned:
+      // 21.9 us with two tiles against 23.7 with one)
       const int want = (a.N + 15) / 16 > cus ? 2 : 1;
       const QmvPlan px = p.NC > 0 && p.NT == want ? QmvPlan{} : plan_qmvx(a.N, a.K, gs, bits, cus);
       if (px.NC > 0 && (p.NC == 0 || px.NT == want)) {
@@ -287,7 +302,15 @@ inline QmmRoute qmm_route(const QmmArgs& a, int gs, int bits, int cus) {
         kernel = QmmKernel::qmvx;
       }
     }
-    if (p.NC > 0) {
+    const KsPlan kp = plan_qmv_ks(a, bits, cus);
+    // (at 8 bits, where the staged kernels don't apply, the streaming kernel too: K = 2560, group
+    // 128, N = 151936, 20 rows 1.35 times; K = 2304, group 64, N = 50176, 17 rows 81.4 us / 71.5)
+    const bool other = p.NC > 0 || (bits == 8 && (gs == 128 || a.M <= 24));
+    if (kp.mt > 0 && !(other && staged_fills_rounds(a.M, a.N, a.K, gs, bits, cus))) {
+      r.kernel = QmmKernel::qmv_ks;
+      r.mt = kp.mt;
+      r.nt = kp.nt;
+    } else if (p.NC > 0) {
       r.kernel = kernel;
       r.mt = mx;
       r.nt = p.NT;

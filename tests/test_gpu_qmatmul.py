@@ -218,6 +218,9 @@ KSPLIT_DECODE = [
     (16, 6144, 2560, 64, 8, "bf16", "qmv 16 2"),
     (3, 40, 12288, 32, 4, "bf16", "qmv 4 1"),
     (17, 40, 14848, 32, 4, "bf16", "qmvx 32 1"),
+    (2, 8213, 2048, 64, 4, "bf16", "qmv 2 1"),          # more columns than one round holds
+    (6, 16390, 2048, 64, 4, "f16", "qmv 8 2"),
+    (24, 8209, 2048, 64, 8, "bf16", "qmv 32 2"),
     (9, 100, 3968, 128, 8, "bf16", "qmm 1 1"),          # 31 groups: the streaming kernel
 ]
 

@@ -547,12 +547,14 @@ int32_t launch_qmv_rows(hipStream_t st, const QmmArgs& a, int mx, const QmvPlan&
 // walks K in chunks of 64, with two roles:
 // - eight compute waves, wave (wm, wn) = (wave % 4, wave / 4) multiplying its 16 MT x 64 block
 //   as MT x 4 16x16x32 MFMA tiles, two k-steps per chunk, from LDS only;
-// - eight loader waves, which load each chunk's x, packed weights, scales and biases three
-//   chunks ahead into registers (three sets in turn), then write x into LDS and dequantise
-//   the weights into it, w = round(fma(s, q, b)) in f32 then to bf16 / f16 (the rounding
-//   of MLX's dequantise, parity unpinned as to one rounding or two). Staging the scales and
-//   biases of all of K in LDS instead was slower over 900 shapes (2 % together, up to 14 %
-//   with 128-row tiles, whose two workgroups per CU the pairs' LDS makes one).
+// - eight loader waves, which load each chunk's x and packed weights three chunks ahead into
+//   registers (three sets in turn), then write x into LDS and dequantise the weights into it,
+//   w = round(fma(s, q, b)) in f32 then to bf16 / f16 (the rounding of MLX's dequantise,
+//   parity unpinned as to one rounding or two). The scales and biases of all of K are staged
+//   in LDS by the compute waves while the first chunks are in flight (2-byte loads of them per
+//   chunk each fetch a cache line: with 256 tiles of 192 rows, K = 4096, 62 us against 58);
+//   where they do not fit beside the buffers or are not 8-byte aligned, the loaders load them
+//   per chunk.
 // Two LDS buffers: the loaders fill chunk c + 1's while the compute waves multiply chunk
 // c's, one barrier per chunk. The loaders issue every load on every path (a chunk past the
 // end loads at offsets past the ranges: zeros, no memory access), so the waits count exactly
@@ -575,7 +577,6 @@ struct Dq {
   static constexpr int kBM = 64 * MT;
   static constexpr uint32_t kXBytes = kBM * 128, kBuf = kXBytes + kDqBN * 128;
   static constexpr uint32_t kLds = 2 * kBuf;  // 96, 80 or 64 KB
-  static_assert(MT > 2 || 2 * kLds <= 160 * 1024, "two workgroups of 128-row tiles per CU");
 };
 
 __device__ __forceinline__ uint32_t dq_unit(uint32_t row, uint32_t u) { return row * 8 + (u ^ ((row >> 1) & 7)); }
@@ -599,7 +600,7 @@ __device__ __forceinline__ uint32_t ld16u(u32x4 rs, uint32_t off) {
   return v;
 }
 
-template <int BITS, int GS, bool F16, int MT>
+template <int BITS, int GS, bool F16, int MT, bool kStaged>
 __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kernel(QmmArgs a, DqPlan p) {
   constexpr int kDqBM = Dq<MT>::kBM;
   constexpr uint32_t kDqXBytes = Dq<MT>::kXBytes, kDqBuf = Dq<MT>::kBuf;
@@ -656,27 +657,48 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
       const uint32_t wo = (w_in ? wr_row * wrow + k0 * BITS / 8 : kOffRow) | no;
       if constexpr (kWq == 2) r.w = ld64(W, wo);
       else r.w = ld128(W, wo);
-      const uint32_t so = (w_in ? wr_row * G2 + 2 * (k0 / GS) : kOffRow) | no;
-      r.s = ld16u(S, so);
-      r.b = ld16u(Bi, so);
+      if constexpr (!kStaged) {
+        const uint32_t so = (w_in ? wr_row * G2 + 2 * (k0 / GS) : kOffRow) | no;
+        r.s = ld16u(S, so);
+        r.b = ld16u(Bi, so);
+      }
     };
-    // loads per chunk: MT of x, 1 of weights, 2 of scales and biases; staging a set waits
-    // for it with the two later sets' loads still in flight
+    // loads per chunk: MT of x, 1 of weights and, unless they are staged, 2 of scales and
+    // biases; staging a set waits for it with the two later sets' loads still in flight
     auto wait_set = [&](Regs& r) __attribute__((always_inline)) {
-      if constexpr (MT == 4)
-        asm volatile("s_waitcnt vmcnt(14)" : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[2]), "+v"(r.x[MT - 1]), "+v"(r.w), "+v"(r.s), "+v"(r.b) : : "memory");
-      else if constexpr (MT == 3)
-        asm volatile("s_waitcnt vmcnt(12)" : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[MT - 1]), "+v"(r.w), "+v"(r.s), "+v"(r.b) : : "memory");
-      else
-        asm volatile("s_waitcnt vmcnt(10)" : "+v"(r.x[0]), "+v"(r.x[MT - 1]), "+v"(r.w), "+v"(r.s), "+v"(r.b) : : "memory");
+      if constexpr (kStaged) {
+        if constexpr (MT == 4)
+          asm volatile("s_waitcnt vmcnt(10)" : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[2]), "+v"(r.x[MT - 1]), "+v"(r.w) : : "memory");
+        else if constexpr (MT == 3)
+          asm volatile("s_waitcnt vmcnt(8)" : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[MT - 1]), "+v"(r.w) : : "memory");
+        else
+          asm volatile("s_waitcnt vmcnt(6)" : "+v"(r.x[0]), "+v"(r.x[MT - 1]), "+v"(r.w) : : "memory");
+      } else {
+        if constexpr (MT == 4)
+          asm volatile("s_waitcnt vmcnt(14)" : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[2]), "+v"(r.x[MT - 1]), "+v"(r.w), "+v"(r.s), "+v"(r.b) : : "memory");
+        else if constexpr (MT == 3)
+          asm volatile("s_waitcnt vmcnt(12)" : "+v"(r.x[0]), "+v"(r.x[1]), "+v"(r.x[MT - 1]), "+v"(r.w), "+v"(r.s), "+v"(r.b) : : "memory");
+        else
+          asm volatile("s_waitcnt vmcnt(10)" : "+v"(r.x[0]), "+v"(r.x[MT - 1]), "+v"(r.w), "+v"(r.s), "+v"(r.b) : : "memory");
+      }
     };
+    const uint32_t* const pairs = reinterpret_cast<const uint32_t*>(smem + 2 * kDqBuf) + wr_row * group_stride(a.G);
     auto stage = [&](Regs& r, int c) __attribute__((always_inline)) {
       const int buf = c & 1;
       wait_set(r);
       uint8_t* const xb = smem + (uint32_t)buf * kDqBuf;
 #pragma unroll
       for (int i = 0; i < MT; ++i) *reinterpret_cast<u32x4*>(xb + 16 * dq_unit(xr0 + 64 * i, xu)) = r.x[i];
-      const float sc = act_to_f32<F16>(r.s), bc = act_to_f32<F16>(r.b);
+      uint32_t sw, bw;
+      if constexpr (kStaged) {
+        const uint32_t sb = pairs[((uint32_t)c * kDqKC + 16 * wh) / GS];
+        sw = sb & 0xffffu;
+        bw = sb >> 16;
+      } else {
+        sw = r.s;
+        bw = r.b;
+      }
+      const float sc = act_to_f32<F16>(sw), bc = act_to_f32<F16>(bw);
       uint8_t* const wb = xb + kDqXBytes;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {  // unit 2 wh + u: k 8 u .. 8 u + 7 of the quarter
@@ -692,6 +714,7 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
     load(0, r0);
     load(1, r1);
     load(2, r2);
+    if constexpr (kStaged) __syncthreads();  // the scales
     stage(r0, 0);
     __syncthreads();
     for (int c = 0; c < NC;) {
@@ -720,6 +743,27 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
   for (int rt = 0; rt < MT; ++rt)
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (kStaged) {
+    // scales and biases of the 128 weight rows into LDS for the loaders, as {scale, bias}
+    // pairs, while these have their first chunks in flight
+    const uint32_t G = (uint32_t)a.G, stride = group_stride(G);
+    const auto S = rsrc(a.s + (int64_t)n0 * G * 2, rows_n * G * 2);
+    const auto Bi = rsrc(a.b + (int64_t)n0 * G * 2, rows_n * G * 2);
+    uint32_t* const pairs = reinterpret_cast<uint32_t*>(smem + 2 * kDqBuf);
+    // a lane takes four groups of a row, a wave `per` rows at a time
+    const uint32_t pieces = G / 4, sh = pieces >= 64 ? 6u : pieces <= 1 ? 0u : 32u - __builtin_clz(pieces - 1);
+    const uint32_t per = 64u >> sh;
+    for (uint32_t row = wave * per + (lane >> sh); row < (uint32_t)kDqBN; row += kDqCompute * per)
+      for (uint32_t g = 4 * (lane & ((1u << sh) - 1)); g < G; g += 256) {
+        const uint32_t off = row < (uint32_t)rows_n ? (row * G + g) * 2 : kOffRow;
+        const u32x2 sv = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(S, off, 0, 0));
+        const u32x2 bv = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(Bi, off, 0, 0));
+        *reinterpret_cast<u32x4*>(pairs + row * stride + g) =
+            u32x4{pair(sv[0], bv[0], kSelLo), pair(sv[0], bv[0], kSelHi), pair(sv[1], bv[1], kSelLo),
+                  pair(sv[1], bv[1], kSelHi)};
+      }
+    __syncthreads();
+  }
   __syncthreads();  // chunk 0 staged
   for (int c = 0; c < NC; ++c) {
     const uint8_t* const xb = smem + (uint32_t)(c & 1) * kDqBuf;
@@ -758,15 +802,24 @@ __global__ __launch_bounds__(64 * (kDqCompute + kDqLoaders)) void qgemm_dq_kerne
       }
 }
 
-template <int BITS, int GS, bool F16, int MT>
-int32_t launch_dq(hipStream_t st, const QmmArgs& a, const DqPlan& p) {
+template <int BITS, int GS, bool F16, int MT, bool kStaged>
+int32_t launch_dq_t(hipStream_t st, const QmmArgs& a, const DqPlan& p, uint32_t lds) {
   static std::atomic<uint64_t> lds_set{0};  // this instantiation's LDS above 64 KB, per device
-  const int32_t rc = allow_lds_once((const void*)qgemm_dq_kernel<BITS, GS, F16, MT>, Dq<MT>::kLds, &lds_set,
+  const int32_t rc = allow_lds_once((const void*)qgemm_dq_kernel<BITS, GS, F16, MT, kStaged>, kQmvMaxLds, &lds_set,
                                     "quantized_matmul: LDS attribute");
   if (rc) return rc;
-  hipLaunchKernelGGL((qgemm_dq_kernel<BITS, GS, F16, MT>), dim3((unsigned)(p.mtiles * p.ntiles)),
-                     dim3(64 * (kDqCompute + kDqLoaders)), Dq<MT>::kLds, st, a, p);
+  hipLaunchKernelGGL((qgemm_dq_kernel<BITS, GS, F16, MT, kStaged>), dim3((unsigned)(p.mtiles * p.ntiles)),
+                     dim3(64 * (kDqCompute + kDqLoaders)), lds, st, a, p);
   return check_hip(hipGetLastError(), "quantized_matmul launch");
+}
+
+template <int BITS, int GS, bool F16, int MT>
+int32_t launch_dq(hipStream_t st, const QmmArgs& a, const DqPlan& p) {
+  // scales through LDS: four groups per 8-byte load, all of K's pairs beside the buffers
+  const uint64_t staged = Dq<MT>::kLds + (uint64_t)kDqBN * group_stride((uint32_t)a.G) * 4;
+  if (a.G % 4 == 0 && (((uintptr_t)a.s | (uintptr_t)a.b) & 7) == 0 && staged <= kQmvMaxLds)
+    return launch_dq_t<BITS, GS, F16, MT, true>(st, a, p, (uint32_t)staged);
+  return launch_dq_t<BITS, GS, F16, MT, false>(st, a, p, Dq<MT>::kLds);
 }
 
 // ---------------------------------------------------------------- one row of x (M = 1)

@@ -226,9 +226,9 @@ KSPLIT_DECODE = [
 
 DQ_TILES = [
     # tiles of 128, 192 and 256 rows of the dequantising GEMM (chosen by the rounds on 256 CUs),
-    # ragged in both directions
+    # ragged in both directions, scales staged in LDS or loaded per chunk (K / gs odd)
     (1020, 4093, 128, 32, 4, "bf16", "qgemm_dq 2 1"),   # 256 tiles of 128 rows
-    (1000, 4096, 192, 64, 8, "f16", "qgemm_dq 2 1"),    # the same, three groups
+    (1000, 4096, 192, 64, 8, "f16", "qgemm_dq 2 1"),    # the same, three groups: loaded per chunk
     (1530, 4090, 256, 32, 8, "bf16", "qgemm_dq 3 1"),   # 256 tiles of 192 rows
     (1531, 4096, 192, 64, 4, "f16", "qgemm_dq 3 1"),
     (2040, 4091, 128, 32, 4, "f16", "qgemm_dq 4 1"),    # 256 tiles of 256 rows
@@ -236,7 +236,8 @@ DQ_TILES = [
 ]
 
 # Scales and biases that start 4 or 2 bytes past a 16-byte boundary (the entry asks for their
-# element's alignment only): the K-split kernels need 8 bytes.
+# element's alignment only): the K-split kernels and the staged scales of the dequantising GEMM
+# need 8 bytes.
 OFF_ALIGNMENT = [
     (20, 6144, 4096, 128, 8, "bf16", 4, "qmvx 32 2"),
     (12, 6144, 4096, 64, 8, "f16", 4, "qmv 16 2"),

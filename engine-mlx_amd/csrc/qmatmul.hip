@@ -550,11 +550,10 @@ int32_t launch_qmv_rows(hipStream_t st, const QmmArgs& a, int mx, const QmvPlan&
 // - eight loader waves, which load each chunk's x and packed weights three chunks ahead into
 //   registers (three sets in turn), then write x into LDS and dequantise the weights into it,
 //   w = round(fma(s, q, b)) in f32 then to bf16 / f16 (the rounding of MLX's dequantise,
-//   parity unpinned as to one rounding or two). The scales and biases of all of K are staged
-//   in LDS by the compute waves while the first chunks are in flight (2-byte loads of them per
-//   chunk each fetch a cache line: with 256 tiles of 192 rows, K = 4096, 62 us against 58);
-//   where they do not fit beside the buffers or are not 8-byte aligned, the loaders load them
-//   per chunk.
+//   parity unpinned as to one rounding or two). From 32 groups on (dq_stages_scales) the
+//   scales and biases of all of K are staged in LDS by the compute waves while the first chunks
+//   are in flight (M = 1531, four layers of 8 bits, K = 4096: 754 us loaded per chunk, 661
+//   staged); else the loaders load them per chunk.
 // Two LDS buffers: the loaders fill chunk c + 1's while the compute waves multiply chunk
 // c's, one barrier per chunk. The loaders issue every load on every path (a chunk past the
 // end loads at offsets past the ranges: zeros, no memory access), so the waits count exactly
@@ -576,7 +575,8 @@ template <int MT>
 struct Dq {
   static constexpr int kBM = 64 * MT;
   static constexpr uint32_t kXBytes = kBM * 128, kBuf = kXBytes + kDqBN * 128;
-  static constexpr uint32_t kLds = 2 * kBuf;  // 96, 80 or 64 KB
+  static constexpr uint32_t kLds = 2 * kBuf;
+  static_assert(kLds == dq_lds(MT), "the plan counts these buffers");
 };
 
 __device__ __forceinline__ uint32_t dq_unit(uint32_t row, uint32_t u) { return row * 8 + (u ^ ((row >> 1) & 7)); }
@@ -815,10 +815,9 @@ int32_t launch_dq_t(hipStream_t st, const QmmArgs& a, const DqPlan& p, uint32_t 
 
 template <int BITS, int GS, bool F16, int MT>
 int32_t launch_dq(hipStream_t st, const QmmArgs& a, const DqPlan& p) {
-  // scales through LDS: four groups per 8-byte load, all of K's pairs beside the buffers
-  const uint64_t staged = Dq<MT>::kLds + (uint64_t)kDqBN * group_stride((uint32_t)a.G) * 4;
-  if (a.G % 4 == 0 && (((uintptr_t)a.s | (uintptr_t)a.b) & 7) == 0 && staged <= kQmvMaxLds)
-    return launch_dq_t<BITS, GS, F16, MT, true>(st, a, p, (uint32_t)staged);
+  if (dq_stages_scales(a, MT))
+    return launch_dq_t<BITS, GS, F16, MT, true>(
+        st, a, p, Dq<MT>::kLds + (uint32_t)kDqBN * group_stride((uint32_t)a.G) * 4);
   return launch_dq_t<BITS, GS, F16, MT, false>(st, a, p, Dq<MT>::kLds);
 }
 

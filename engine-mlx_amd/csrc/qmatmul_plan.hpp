@@ -55,6 +55,19 @@ struct DqPlan {
 // so that the arithmetic of a call does not depend on which of them its sizes choose.
 inline bool dq_x_fits(int64_t ldx, int K) { return 256 * ldx * 2 + (int64_t)K * 2 < ((int64_t)1 << 31); }
 
+// LDS of its two buffers (x and weight rows of a chunk): 96, 80 or 64 KB.
+constexpr uint32_t dq_lds(int mt) { return 2 * (64 * mt + kDqBN) * 128; }
+
+// Whether the dequantising GEMM stages all of K's scales and biases in LDS: from 32 groups a row
+// on. Loaded per chunk, their 2-byte loads each fetch a cache line, so with the weights in HBM
+// staging is 7 to 22 % faster at 64 groups and 0 to 4 % at 32; at 8 to 24 it is up to 3 % slower,
+// for its barrier ahead of the first chunk, and 128-row tiles, two workgroups of which share a CU,
+// gain nothing from the pairs' LDS. Four groups per 8-byte load, all pairs beside the buffers.
+inline bool dq_stages_scales(const QmmArgs& a, int mt) {
+  return a.G >= 32 && a.G % 4 == 0 && (((uintptr_t)a.s | (uintptr_t)a.b) & 7) == 0 &&
+         dq_lds(mt) + (uint64_t)kDqBN * group_stride((uint32_t)a.G) * 4 <= 160 * 1024;
+}
+
 // Plan of the dequantising GEMM: K a multiple of the chunk and of the group, x within one
 // buffer range per tile. Regions: 2 x 4, 4 x 2, 1 x 8 or 8 x 1 whole tile rows and columns,
 // the one with the least bytes per region, when the grid divides into them.

@@ -1,7 +1,7 @@
 // Prints which kernel and tiles a quantised projection takes, by the rules that the launches
 // use (engine-mlx_amd/csrc/qmatmul_plan.hpp): one line "kernel mt nt" per input line
-// "M N K group bits ldx scale_offset cus" (scale_offset: bytes of scales and biases past a
-// 16-byte boundary).
+// "M N K group bits ldx scale_offset cus" (scale_offset: bytes of scales and biases past a 16-byte
+// boundary; qgemm_dq_staged: qgemm_dq with its scales through LDS).
 #include <cstdio>
 
 #include "qmatmul_plan.hpp"
@@ -18,7 +18,8 @@ int main() {
     a.K = (int)k;
     a.G = (int)(k / gs);
     const ema::QmmRoute r = ema::qmm_route(a, (int)gs, (int)bits, (int)cus);
-    std::printf("%s %d %d\n", names[(int)r.kernel], r.mt, r.nt);
+    const bool staged = r.kernel == ema::QmmKernel::qgemm_dq && ema::dq_stages_scales(a, r.mt);
+    std::printf("%s%s %d %d\n", names[(int)r.kernel], staged ? "_staged" : "", r.mt, r.nt);
   }
   return 0;
 }

@@ -226,13 +226,19 @@ KSPLIT_DECODE = [
 
 DQ_TILES = [
     # tiles of 128, 192 and 256 rows of the dequantising GEMM (chosen by the rounds on 256 CUs),
-    # ragged in both directions, scales staged in LDS or loaded per chunk (K / gs odd)
+    # ragged in both directions, scales loaded per chunk and, from 32 groups on, staged in LDS
     (1020, 4093, 128, 32, 4, "bf16", "qgemm_dq 2 1"),   # 256 tiles of 128 rows
-    (1000, 4096, 192, 64, 8, "f16", "qgemm_dq 2 1"),    # the same, three groups: loaded per chunk
+    (1000, 4096, 192, 64, 8, "f16", "qgemm_dq 2 1"),    # the same, three groups
     (1530, 4090, 256, 32, 8, "bf16", "qgemm_dq 3 1"),   # 256 tiles of 192 rows
     (1531, 4096, 192, 64, 4, "f16", "qgemm_dq 3 1"),
     (2040, 4091, 128, 32, 4, "f16", "qgemm_dq 4 1"),    # 256 tiles of 256 rows
     (2047, 4096, 64, 64, 8, "bf16", "qgemm_dq 4 1"),    # one chunk
+    (80, 64, 1152, 64, 4, "bf16", "qgemm_dq 2 1"),      # 18 groups: not the K-split kernel
+    (1020, 4093, 1024, 32, 4, "bf16", "qgemm_dq_staged 2 1"),
+    (1530, 4090, 1024, 32, 8, "bf16", "qgemm_dq_staged 3 1"),
+    (1531, 4096, 2048, 64, 4, "f16", "qgemm_dq_staged 3 1"),
+    (2040, 4091, 1024, 32, 4, "f16", "qgemm_dq_staged 4 1"),
+    (2047, 4096, 2048, 64, 8, "bf16", "qgemm_dq_staged 4 1"),
 ]
 
 # Scales and biases that start 4 or 2 bytes past a 16-byte boundary (the entry asks for their
@@ -242,8 +248,8 @@ OFF_ALIGNMENT = [
     (20, 6144, 4096, 128, 8, "bf16", 4, "qmvx 32 2"),
     (12, 6144, 4096, 64, 8, "f16", 4, "qmv 16 2"),
     (32, 4096, 4096, 64, 8, "bf16", 4, "qmv 32 1"),
-    (157, 4093, 1024, 64, 4, "bf16", 4, "qgemm_dq 2 1"),
-    (157, 300, 1024, 64, 8, "f16", 2, "qgemm_dq 2 1"),
+    (157, 4093, 2048, 64, 4, "bf16", 4, "qgemm_dq 2 1"),
+    (157, 300, 2048, 64, 8, "f16", 2, "qgemm_dq 2 1"),
 ]
 
 

@@ -265,25 +265,27 @@ inline int qmv_rows(int M) { return M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 
 inline bool gemv1_fits(int G, int K) { return (G % 64 == 0 || (G <= 64 && (G & (G - 1)) == 0)) && K <= 32768; }
 
 // Up to 32 rows, K of 2048 to 3072 and more columns than one round of workgroups holds: whether
-// the kernels that keep a column tile's weights in LDS (one to three chunks at such K) are faster
-// than the K-split kernel, each of whose waves has two or three units per workgroup to set against
-// its fixed 3.5 us. r1, r2: rounds of workgroups with one and two column tiles each (K-split: one;
-// the staged kernel: one up to 4 rows, two above, so that it gains where r2 is just full).
-// Measured, us, K-split / staged, 4 bits, group 64: K = 2048, N = 151936 81.5 / 54.9 at 2 rows,
-// 85.0 / 59.1 at 8; N = 16384 18.7 / 17.0 at 24; N = 9216 at 24 1.13 times faster split. 8 bits: K =
-// 2048, N = 32768, 32 rows 51.5 / 37.2; K = 2560 60.2 / 48.2. From K = 4096 on it is faster at
-// every N.
-inline bool staged_fills_rounds(int M, int N, int K, int gs, int bits, int cus) {
+// the kernels that keep a column tile's weights in LDS (`staged`: one to three chunks at such K)
+// are faster than the K-split kernel, each of whose waves has two or three units per workgroup to
+// set against its fixed 3.5 us. r1, r2: rounds of workgroups with one and two column tiles each
+// (K-split: one; the staged kernels: one up to 4 rows, two above, so that they gain most where
+// the two-tile rounds are full). Where they don't apply, 8 bits leave the streaming kernel.
+// Measured with the weights in HBM, us, K-split / the other, group 64, K = 2048, 4 bits: N = 151936
+// 81.4 / 55.2 at 2 rows, N = 32768 38.3 / 32.0 at 24, N = 9216 15.3 / 16.3 at 24; 8 bits, N =
+// 32768, 32 rows 56.8 / 39.1. K = 2560, 32 rows: 8 bits, N = 32768 62.0 / 49.3; 4 bits, N = 9216
+// 17.6 / 22.7. From K = 4096 on the K-split kernel is faster at every N.
+inline bool staged_fills_rounds(int M, int N, int K, int gs, int bits, int cus, bool staged) {
   const int t1 = (N + 15) / 16, t2 = (N + 31) / 32;
   if (t2 <= cus) return false;
   const int r1 = (t1 + cus - 1) / cus, r2 = (t2 + cus - 1) / cus;
   const bool even = r1 >= 2 * r2 || r1 > 12;
-  if (M <= 2) return r1 > (K <= 2048 ? 2 : K == 2560 ? 20 : K == 3072 ? 6 : N);
-  if (M <= 4) return K <= 2048 && r1 > 3;
-  if (M <= 8) return K <= 2048 && r1 > 3;
-  if (M <= 16) return K <= 2048 && gs >= 64 && even;
-  if (bits == 4) return K <= 2048 ? (gs == 32 ? r1 > 3 : even) : K <= 3072 && gs == 32 && even;
-  return K <= 2048 || (K <= 2560 && r1 > (gs == 128 ? 2 : 3)) || (K <= 3072 && gs <= 64 && r1 > 7 && even);
+  if (!staged) return bits == 8 && M > 16 && (K == 2560 || (K <= 2304 && M <= 24 && r1 > 3));
+  if (M <= 2) return K <= 2048 || (K == 2560 && r1 > 8) || (K == 3072 && (gs > 32 || r1 > 6));
+  if (M <= 4) return K <= 2048 || (K == 3072 && gs == 128);
+  if (M <= 8) return K <= 2048 && r1 > (gs == 32 ? 3 : 2);
+  if (M <= 16) return K <= 2048 && gs > 32 && (even || r1 > 6);
+  if (bits == 4) return K <= 2048 ? r1 > (gs == 32 && M <= 24 ? 2 : 3) : K <= 3072 && gs == 32 && even;
+  return K <= 2048 || (K <= 2560 && r1 > (K == 2560 && M <= 24 ? 2 : 3)) || (K <= 3072 && even);
 }
 
 enum class QmmKernel { gemv1, qmv_ks, qgemm_ks, qmv, qmvx, qgemm_dq, qmm };
@@ -316,10 +318,7 @@ inline QmmRoute qmm_route(const QmmArgs& a, int gs, int bits, int cus) {
       }
     }
     const KsPlan kp = plan_qmv_ks(a, bits, cus);
-    // (at 8 bits, where the staged kernels don't apply, the streaming kernel too: K = 2560, group
-    // 128, N = 151936, 20 rows 1.35 times; K = 2304, group 64, N = 50176, 17 rows 81.4 us / 71.5)
-    const bool other = p.NC > 0 || (bits == 8 && (gs == 128 || a.M <= 24));
-    if (kp.mt > 0 && !(other && staged_fills_rounds(a.M, a.N, a.K, gs, bits, cus))) {
+    if (kp.mt > 0 && !staged_fills_rounds(a.M, a.N, a.K, gs, bits, cus, p.NC > 0)) {
       r.kernel = QmmKernel::qmv_ks;
       r.mt = kp.mt;
       r.nt = kp.nt;

@@ -129,8 +129,12 @@ __device__ __forceinline__ uint32_t pk_max3_f16(uint32_t a, uint32_t b, uint32_t
 // workgroup instead of two, and no refill of the pipeline between the blocks. The light
 // rows are complete when group 0 leaves them; group 0 stores them on its own. A middle
 // block paired with itself (odd block count) runs as a heavy block with no light rows.
-template <bool kRot, bool kPair>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_kernel(PrefillArgs a) {
+// kWindow (with kPair): chunk-only calls, whose window may begin inside a key block.
+// Aligned, since the time of a kernel this long depends on where its code lies (T 2048, 32q/8kv
+// with its pre-attention: 51.6 us from a 4 KB boundary, 51.8 to 52.3 at other multiples of 256).
+template <bool kRot, bool kPair, bool kWindow = false>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2), aligned(4096))) void prefill_kernel(
+    PrefillArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
 
   const int tid = threadIdx.x;
@@ -218,7 +222,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     return kSeg == 1 || (kSeg == 0 && kPair && j < n1);
   };
   const int offB = gbB - n1;
-  const int n1_edge = kPair && kv_begin % kBN ? n1 - 2 : n1;
+  const int n1_edge = kWindow && kv_begin % kBN ? n1 - 2 : n1;
   auto blk_of = [&](int j) __attribute__((always_inline)) { return j + (in_a(j, SegAny{}) ? gbA : offB); };
 
   const int hh = lane >> 5;                       // which half of the k slots
@@ -497,7 +501,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       // inf or NaN, which the maximum keeps.
       // (not in segment A's last steps when a window begins inside a block: they load segment
       // B's first block, that block again, and only load_k / load_v leave out its early rows)
-      bool fast = all_seen && !(kMask && decltype(seg)::value == 1 && j >= n1_edge);
+      bool fast = all_seen && !(kWindow && kMask && decltype(seg)::value == 1 && j >= n1_edge);
       if (fast) {
         const uint32_t kob = blk_off(j + 2), vob = blk_off(j + 1);
         const int kwrap = wrap_rows(j + 2), vwrap = wrap_rows(j + 1);
@@ -641,7 +645,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       const uint16_t* qp = light_q(32 * wq) + k_lane;
       for (int s = 0; s < 8; ++s) qop[s] = scale_q(*(const u32x4*)(qp + (k_x ^ (16 * s))));
       const int actA = seg_act(gbA, wfaA, n1), maskA = seg_mask(gbA, wfaA);
-      const int tfA = actA < maskA ? (actA < n1_edge ? actA : n1_edge) : (maskA < n1_edge ? maskA : n1_edge);
+      int tfA = actA < maskA ? actA : maskA;
+      if (kWindow && tfA > n1_edge) tfA = n1_edge;
       for (; t < n1 - 1 && t < 1; ++t) half0(t, false, mask_on, SegA{}, false);
       for (; t < n1 - 1 && t < tfA; ++t) half0(t, true, mask_off, SegA{}, false);
       for (; t < n1 - 1; ++t) half0(t, false, mask_on, SegA{}, false);
@@ -968,10 +973,11 @@ int32_t launch_prefill(hipStream_t s, const void* q, const ema_kvcache_desc& c,
     return set_error(EMA_ERR_UNSUPPORTED,
                      "ema_prefill_attention: capacity %d x stride_pos %lld exceeds the 2 GiB per-head range",
                      c.capacity, (long long)c.stride_pos);
-  static std::atomic<uint64_t> lds_set[4];  // per instantiation, one bit per device
-  const void* kernels[4] = {(const void*)prefill_kernel<false, false>, (const void*)prefill_kernel<true, false>,
-                            (const void*)prefill_kernel<false, true>, (const void*)prefill_kernel<true, true>};
-  for (int i = 0; i < 4; ++i) {
+  static std::atomic<uint64_t> lds_set[6];  // per instantiation, one bit per device
+  const void* kernels[6] = {(const void*)prefill_kernel<false, false>, (const void*)prefill_kernel<true, false>,
+                            (const void*)prefill_kernel<false, true>, (const void*)prefill_kernel<true, true>,
+                            (const void*)prefill_kernel<false, true, true>, (const void*)prefill_kernel<true, true, true>};
+  for (int i = 0; i < 6; ++i) {
     const int32_t rc = allow_lds_once(kernels[i], kLdsBytes, &lds_set[i], "ema_prefill_attention: LDS attribute");
     if (rc) return rc;
   }
@@ -1014,7 +1020,12 @@ int32_t launch_prefill(hipStream_t s, const void* q, const ema_kvcache_desc& c,
   a.paired = a.nqb >= 2 && items >= 2 * (int64_t)cus;
   const int64_t blocks = prefill_grid(c.batch, Hq, a.nqb, a.paired);
   if (blocks > 0x7fffffff) return set_error(EMA_ERR_SHAPE, "ema_prefill_attention: grid too large");
-  if (rot && a.paired)
+  const bool window = flags & EMA_PREFILL_CHUNK_ONLY;
+  if (rot && a.paired && window)
+    hipLaunchKernelGGL((prefill_kernel<true, true, true>), dim3((unsigned)blocks), dim3(kThreads), kLdsBytes, s, a);
+  else if (a.paired && window)
+    hipLaunchKernelGGL((prefill_kernel<false, true, true>), dim3((unsigned)blocks), dim3(kThreads), kLdsBytes, s, a);
+  else if (rot && a.paired)
     hipLaunchKernelGGL((prefill_kernel<true, true>), dim3((unsigned)blocks), dim3(kThreads), kLdsBytes, s, a);
   else if (rot)
     hipLaunchKernelGGL((prefill_kernel<true, false>), dim3((unsigned)blocks), dim3(kThreads), kLdsBytes, s, a);

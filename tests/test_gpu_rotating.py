@@ -190,7 +190,13 @@ def test_rotating_prefill_paired(ema, ora, q_off, chunk):
     big_k = ora.normal_bf16((B, Hkv, int(L.max()), D), seed=71)
     big_v = ora.normal_bf16((B, Hkv, int(L.max()), D), seed=72)
     q = ora.normal_bf16((B, Hq, T, D), seed=73)
-    cache = ring_cache(ema, ring_from(ora, big_k, L, W), ring_from(ora, big_v, L, W))
+    ring_k, ring_v = ring_from(ora, big_k, L, W), ring_from(ora, big_v, L, W)
+    if chunk:  # rows before the chunk are never read
+        for b in range(B):
+            for r, p in ora.ring_rows(int(L[b]), W).items():
+                if p < qo[b]:
+                    ring_k[b, :, r] = ring_v[b, :, r] = NAN
+    cache = ring_cache(ema, ring_k, ring_v)
     out = ema.prefill_attention(dev(q), cache, dev(qo), causal=True, chunk_only=chunk)
     torch.cuda.synchronize()
     lo = np.maximum(L - W, 0)

@@ -49,12 +49,19 @@ int device_cus() {
   return n;
 }
 
-int32_t allow_lds_once(const void* fn, int bytes, std::atomic<uint64_t>* done, const char* what) {
+int32_t allow_lds_once(const void* const* fns, int n, int bytes, std::atomic<uint64_t>* done, const char* what) {
   const uint64_t bit = 1ull << current_device();
   if (done->load(std::memory_order_acquire) & bit) return EMA_OK;
-  const int32_t rc = check_hip(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes), what);
-  if (rc == EMA_OK) done->fetch_or(bit, std::memory_order_release);
-  return rc;
+  for (int i = 0; i < n; ++i) {
+    const int32_t rc = check_hip(hipFuncSetAttribute(fns[i], hipFuncAttributeMaxDynamicSharedMemorySize, bytes), what);
+    if (rc) return rc;
+  }
+  done->fetch_or(bit, std::memory_order_release);
+  return EMA_OK;
+}
+
+int32_t allow_lds_once(const void* fn, int bytes, std::atomic<uint64_t>* done, const char* what) {
+  return allow_lds_once(&fn, 1, bytes, done, what);
 }
 
 }  // namespace ema

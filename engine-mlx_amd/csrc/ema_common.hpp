@@ -178,6 +178,8 @@ int device_cus();
 // Raises `fn`'s dynamic LDS limit to `bytes` once per device; bit d of *done records
 // device d (thread-safe).
 int32_t allow_lds_once(const void* fn, int bytes, std::atomic<uint64_t>* done, const char* what);
+// The same for n kernels.
+int32_t allow_lds_once(const void* const* fns, int n, int bytes, std::atomic<uint64_t>* done, const char* what);
 // Maps a HIP error to EMA_ERR_HIP with context, or returns EMA_OK.
 int32_t check_hip(hipError_t e, const char* what);
 

@@ -273,7 +273,7 @@ template <int DK, int kScanWaves>
 struct ScanLds {
   static constexpr int kV = Rec<DK>::kU;        // the value-head record up to u
   static constexpr int kK = kV;                 // then the key-head record
-  static constexpr int kU = kK + Rec<DK>::kKey; // then u of the workgroup's four row blocks
+  static constexpr int kU = kK + Rec<DK>::kKey; // then u of the workgroup's row blocks, one per wave
   static constexpr int kBuf = kU + kScanWaves * 2048;
   static constexpr int kBytes = 3 * kBuf;
   static constexpr int kDma = (kBuf) / 1024;    // 1 KB steps per chunk

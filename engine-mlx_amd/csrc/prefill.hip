@@ -973,14 +973,17 @@ int32_t launch_prefill(hipStream_t s, const void* q, const ema_kvcache_desc& c,
     return set_error(EMA_ERR_UNSUPPORTED,
                      "ema_prefill_attention: capacity %d x stride_pos %lld exceeds the 2 GiB per-head range",
                      c.capacity, (long long)c.stride_pos);
-  static std::atomic<uint64_t> lds_set[6];  // per instantiation, one bit per device
-  const void* kernels[6] = {(const void*)prefill_kernel<false, false>, (const void*)prefill_kernel<true, false>,
-                            (const void*)prefill_kernel<false, true>, (const void*)prefill_kernel<true, true>,
-                            (const void*)prefill_kernel<false, true, true>, (const void*)prefill_kernel<true, true, true>};
-  for (int i = 0; i < 6; ++i) {
-    const int32_t rc = allow_lds_once(kernels[i], kLdsBytes, &lds_set[i], "ema_prefill_attention: LDS attribute");
-    if (rc) return rc;
-  }
+  // every kernel's LDS above 64 KB at once: one look at the device per call, not one per kernel
+  // (the smallest calls are bound by the host)
+  static std::atomic<uint64_t> lds_set;  // one bit per device
+  const void* const kernels[8] = {
+      (const void*)prefill_kernel<false, false>,      (const void*)prefill_kernel<true, false>,
+      (const void*)prefill_kernel<false, true>,       (const void*)prefill_kernel<true, true>,
+      (const void*)prefill_kernel<false, true, true>, (const void*)prefill_kernel<true, true, true>,
+      (const void*)prefill_few_kernel<false>,         (const void*)prefill_few_kernel<true>};
+  const int32_t rc = allow_lds_once(kernels, 8, kLdsBytes > kFewLds ? kLdsBytes : kFewLds, &lds_set,
+                                    "ema_prefill_attention: LDS attribute");
+  if (rc) return rc;
   PrefillArgs a;
   a.q = (const uint16_t*)q;
   a.k = (const uint16_t*)c.k;
@@ -1002,10 +1005,6 @@ int32_t launch_prefill(hipStream_t s, const void* q, const ema_kvcache_desc& c,
   const int cus = device_cus();
   const bool rot = c.flags & EMA_KV_ROTATING;
   if (prefill_few(c.batch, Hq, T, cus)) {
-    static std::atomic<uint64_t> few_set[2];
-    const void* fk = rot ? (const void*)prefill_few_kernel<true> : (const void*)prefill_few_kernel<false>;
-    const int32_t rc = allow_lds_once(fk, kFewLds, &few_set[rot ? 1 : 0], "ema_prefill_attention: LDS attribute");
-    if (rc) return rc;
     a.nqb = prefill_few_blocks(T);
     a.paired = 0;
     const int64_t blocks = prefill_grid(c.batch, Hq, a.nqb, 0);

@@ -961,9 +961,10 @@ int32_t launch_gemv1(hipStream_t st, const QmmArgs& a, int cus) {
 
 template <int BITS, int GS, bool F16>
 int32_t launch_t(hipStream_t st, QmmArgs a) {
-  const QmmRoute r = qmm_route(a, GS, BITS, device_cus());
+  const int cus = device_cus();
+  const QmmRoute r = qmm_route(a, GS, BITS, cus);
   switch (r.kernel) {
-    case QmmKernel::gemv1: return launch_gemv1<BITS, GS, F16>(st, a, device_cus());
+    case QmmKernel::gemv1: return launch_gemv1<BITS, GS, F16>(st, a, cus);
     case QmmKernel::qmv_ks: return launch_qmv_ks(st, a, KsPlan{r.mt, r.nt}, GS, BITS, F16);
     case QmmKernel::qgemm_ks: return launch_qgemm_ks(st, a, KsPlan{r.mt, r.nt}, GS, BITS, F16);
     case QmmKernel::qmv: return launch_qmv_rows<BITS, GS, F16>(st, a, r.mt, r.qmv);

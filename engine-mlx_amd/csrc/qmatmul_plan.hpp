@@ -122,9 +122,12 @@ inline bool ks_fits(const QmmArgs& a) {
 // = 2048 and 4096, in units of 25 ns: a workgroup takes 140 and, per turn of its eight waves
 // over a unit each, 4 + 16 per row tile + 18 per column tile (qgemm_dq_kernel: dq_cost; K =
 // 4096, N = 4096: 33 us here against 45 at 300 rows, 45 against 45 at 520, 58 against 46 at
-// 700). The column tiles of an XCD all read all of x, so it has to stay in its 4 MB L2: K = 2048,
-// N = 1024 21.5 us here against 24 at 1200 rows (4.7 MB), 25.1 against 24.5 at 1531 (6 MB) and
-// 39.9 against 23.8 at 2048 (8 MB).
+// 700). The column tiles of an XCD all read all of x, and past its 4 MB L2 they read it from
+// further off; the line at 5 MB was measured at K = 2048, N = 1024: 21.5 us here against 24 at 1200
+// rows (4.7 MB), 25.1 against 24.5 at 1531 (6 MB) and 39.9 against 23.8 at 2048 (8 MB). It does not
+// hold everywhere: with K >= 3072, N <= 2048 and x of 5 to 8 MB this kernel would still be the
+// faster one (K = 4096, N = 1024, 700 rows 17.3 us against 42.1), with N >= 4096 it is not (600 rows
+// 54 against 44).
 inline KsPlan plan_ks(const QmmArgs& a, int bits, int cus) {
   KsPlan best{0, 0};
   if (!ks_fits(a) || !dq_x_fits(a.ldx, a.K) || (int64_t)a.M * a.K * 2 > (5 << 20)) return best;

@@ -14,10 +14,12 @@
 // Two regimes, as in MLX, whose quantized matmul takes vector kernels for a few rows of x
 // and, for many, kernels that dequantise weight tiles into the activation type first:
 // - up to 32 rows (and the streaming fallback): exact products, below, and qgemm_ks.hip from
-//   K = 2048 on (8 bits and up to 16 rows: from K = 4096 on);
+//   K = 2048 on (8 bits and up to 16 rows: from K = 4096 on), except for some calls of many
+//   columns;
 // - more than 32 rows with K a multiple of 64: qgemm_dq_kernel, and the K-split kernel of
 //   qgemm_ks.hip where small tiles fill the chip better, on weights dequantised into bf16 /
 //   f16 (one rounding each).
+// The rules are in qmatmul_plan.hpp (qmm_route).
 //
 // Exact products. The MFMA's B operand is not the dequantised weight (which would have to
 // be rounded to bf16) but C + q, with the field's bits dropped into the mantissa of the
